@@ -167,6 +167,8 @@ typedef struct {
     float* partials_b; /* 3*M, as partials */
     const uint32_t* tile_range; /* node-fused steps: ntiles*MX*2, for tile-node j of tile c the range
                                    [node_off[n], node_off[n+1]) of its node n's partials at 2*(c*MX + j) */
+    int32_t tile_odd;  /* NFX_SCATTER_TILED without the node-fused buffers: 1 = nfx_order_tiles_host has ordered the
+                          tile arrays (run starts at odd distances); 0 = as nfx_build_tiles_host filled them */
 } nfx_plan;
 
 /* Per-cell parameters of a batch, in that cell's simulation units.  The batched material is the
@@ -282,6 +284,14 @@ int nfx_gather_corners(nfx_ctx* ctx, const uint32_t* csr_offsets, const uint32_t
 int nfx_build_tiles_host(const uint32_t* tetras_host, int64_t N, int64_t T, int32_t tile_k, int32_t* max_nodes,
                          int64_t* m_total, uint32_t* tile_count, uint32_t* tile_nodes, uint16_t* tile_lend,
                          uint16_t* tile_corners, uint32_t* tile_dst, uint32_t* node_off);
+/* Orders the tile-nodes of every tile by descending run length (equal lengths keep their order), in place in
+ * tile_nodes, tile_lend, tile_corners and tile_dst as nfx_build_tiles_host filled them, and lets every run of
+ * the corner list start an odd distance after the one before it: tile_lend then holds the runs' ends in that
+ * list, where run j starts at the first place of j's parity at or after the end of run j - 1.  perm (ntiles*MX):
+ * the old index of each tile-node.  Set nfx_plan.tile_odd for arrays in this form. */
+int nfx_order_tiles_host(int64_t ntiles, int32_t tile_k, int32_t max_nodes, const uint32_t* tile_count,
+                         uint32_t* tile_nodes, uint16_t* tile_lend, uint16_t* tile_corners, uint32_t* tile_dst,
+                         uint16_t* perm);
 /* host-side CSR build (host pointers): offsets N+1, slots 4T ascending per node */
 int nfx_build_node_csr_host(const uint32_t* tetras_host, int64_t N, int64_t T, uint32_t* offsets_host,
                             uint32_t* slots_host);

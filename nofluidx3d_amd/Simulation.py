@@ -66,6 +66,18 @@ def tile_ranges(tile_nodes, count, node_off, max_nodes):
     return out.reshape(-1)
 
 
+def order_tiles(tile_k, max_nodes, count, arrays):
+    """Order host tile arrays (tile_nodes, tile_lend, tile_corners, tile_dst) as plan.tile_odd takes them, in place
+    (nfx_order_tiles_host); returns the old index of each tile-node (ntiles x max_nodes)."""
+    import ctypes
+
+    vp = ctypes.c_void_p
+    perm = np.zeros((len(count), max_nodes), np.uint16)
+    _lib.call("nfx_order_tiles_host", len(count), tile_k, max_nodes, count.ctypes.data_as(vp),
+              *[a.ctypes.data_as(vp) for a in arrays], perm.ctypes.data_as(vp))
+    return perm
+
+
 class Simulation:
     def __init__(self, con, scatter="tiled", fused=True, use_graph=True, mesh=None, verbose=True, tile_k=512,
                  stream_nt=None, shape_from_ref=True, fuse_node_pass=None):
@@ -506,18 +518,13 @@ class Simulation:
                       node_off.ctypes.data_as(vp))
             dev = self.device
             to = lambda a: torch.from_numpy(a.view(np.int32) if a.dtype == np.uint32 else a.view(np.int16)).to(dev)
-            tile_range = tile_ranges(tile_nodes, count, node_off, MX)
             self._tiles = {
                 "tile_k": K,
                 "max_nodes": MX,
                 "m_total": M,
+                "host": (count, node_off, tile_nodes, tile_lend, tile_corners, tile_dst),
                 "tile_count": to(count),
-                "tile_nodes": to(tile_nodes),
-                "tile_lend": to(tile_lend),
-                "tile_corners": to(tile_corners),
-                "tile_dst": to(tile_dst),
                 "node_off": to(node_off),
-                "tile_range": to(tile_range),
                 "partials": torch.zeros(3 * M, dtype=torch.float32, device=dev),
                 # every node is a corner of some tetra (has a partial): the node-fused step updates
                 # nodes only through the tiles that touch them
@@ -525,6 +532,26 @@ class Simulation:
             }
             torch.cuda.synchronize(dev)
         return self._tiles
+
+    def tile_lists(self, node_fused):
+        """The per-tile node and corner lists on the device: as built, with the nodes' partial ranges, for
+        node-fused steps, else in the order of ``order_tiles``."""
+        t = self.node_tiles()
+        key = "fused" if node_fused else "ordered"
+        if key not in t:
+            import torch
+
+            K, MX = t["tile_k"], t["max_nodes"]
+            count, node_off, *lists = t["host"]
+            to = lambda a: torch.from_numpy(a.view(np.int32) if a.dtype == np.uint32 else a.view(np.int16)).to(self.device)
+            if not node_fused:
+                lists = [a.copy() for a in lists]
+                order_tiles(K, MX, count, lists)
+            t[key] = {k: to(a) for k, a in zip(("tile_nodes", "tile_lend", "tile_corners", "tile_dst"), lists)}
+            if node_fused:
+                t[key]["tile_range"] = to(tile_ranges(lists[0], count, node_off, MX))
+            torch.cuda.synchronize(self.device)
+        return t[key]
 
     def plan(self):
         """The fused-step description of the registered plugin chain, or None if it cannot fuse.
@@ -605,10 +632,15 @@ class Simulation:
                     self._vp_active = torch.ones(ntiles, dtype=torch.int32, device=self.device)
                 p.vp_active = self._vp_active.data_ptr()
                 self._vp_flags_stale = True
-            for k in ("tile_count", "tile_nodes", "tile_lend", "tile_corners", "tile_dst", "node_off", "partials"):
+            fuse = self.node_fused_wanted() and t["every_node"] and p.model in (_lib.NFX_SVKK, _lib.NFX_SVK, _lib.NFX_MR,
+                                                                                _lib.NFX_VISCOPLASTIC)
+            lists = self.tile_lists(fuse)
+            for k in ("tile_count", "node_off", "partials"):
                 setattr(p, k, t[k].data_ptr())
-            if self.node_fused_wanted() and t["every_node"] and p.model in (_lib.NFX_SVKK, _lib.NFX_SVK, _lib.NFX_MR,
-                                                                        _lib.NFX_VISCOPLASTIC):
+            for k, a in lists.items():
+                setattr(p, k, a.data_ptr())
+            p.tile_odd = 0 if fuse else 1
+            if fuse:
                 import torch
 
                 if self._node_b is None:
@@ -617,7 +649,6 @@ class Simulation:
                     t["partials_b"] = torch.zeros_like(t["partials"])
                 p.disp_b, p.vel_b = self._node_b[0].data_ptr(), self._node_b[1].data_ptr()
                 p.partials_b = t["partials_b"].data_ptr()
-                p.tile_range = t["tile_range"].data_ptr()
         else:
             p.scatter = _lib.SCATTER_ATOMIC
         self._plan, self._plan_key = p, key

@@ -103,6 +103,7 @@ class Plan(ctypes.Structure):
         ("vel_b", c_vp),
         ("partials_b", c_vp),
         ("tile_range", c_vp),
+        ("tile_odd", c_i32),
     ]
 
 
@@ -198,6 +199,7 @@ SIGNATURES = {
     "nfx_build_node_csr_host": (ctypes.c_int, [c_vp, c_i64, c_i64, c_vp, c_vp]),
     "nfx_build_tiles_host": (ctypes.c_int, [c_vp, c_i64, c_i64, c_i32, ctypes.POINTER(c_i32), ctypes.POINTER(c_i64),
                                             c_vp, c_vp, c_vp, c_vp, c_vp, c_vp]),
+    "nfx_order_tiles_host": (ctypes.c_int, [c_i64, c_i32, c_i32, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp]),
     "nfx_sphere_force": (ctypes.c_int, [c_vp, c_vp, c_vp, c_i64, c_f64, c_f64, c_f64]),
     "nfx_substrate_force": (ctypes.c_int, [c_vp, c_vp, c_vp, c_i64, c_f64, c_f64]),
     "nfx_plane_force": (ctypes.c_int, [c_vp, c_vp, c_vp, c_i64, c_f64, c_f64]),

@@ -32,6 +32,7 @@ import numpy as np
 
 from nofluidx3d_amd import _lib
 from nofluidx3d_amd.autotune import default_stream_nt
+from nofluidx3d_amd.Simulation import order_tiles
 
 E_SIM = 1e-2
 
@@ -323,6 +324,16 @@ def build_host_arrays(specs, meshes, steps, tile_k):
     return h
 
 
+def order_batch_tiles(h, tile_k):
+    """The tile arrays of ``build_host_arrays`` in the order the device step takes them (order_tiles), in place."""
+    MX = h["max_nodes"]
+    perm = order_tiles(tile_k, MX, h["tile_count"],
+                       [h[k] for k in ("tile_nodes", "tile_lend", "tile_corners", "tile_dst")]).astype(np.int64)
+    for k in ("tile_nodes16", "tile_dst16"):
+        if k in h:
+            h[k] = np.take_along_axis(h[k].reshape(-1, MX), perm, 1).reshape(-1)
+
+
 class BatchSimulation:
     """All cells of ``specs`` on the current device.  ``meshes``: list of (points_um, tets).
 
@@ -358,6 +369,7 @@ class BatchSimulation:
             raise ValueError("a batch is either all elastic or all viscoplastic")
         self.model = _lib.NFX_VISCOPLASTIC if viscous[0] else _lib.NFX_MR
         h = build_host_arrays(specs, meshes, steps, K)
+        order_batch_tiles(h, K)
         self._meshes = meshes
         self.cells_host, self.units, self.radius_sim = h["cells"], h["units"], h["radius_sim"]
         self.node_off, self.tet_pad_off = h["node_off"], h["tet_pad_off"]
@@ -434,7 +446,7 @@ class BatchSimulation:
         p.stream_nt = default_stream_nt(self.T) if stream_nt is None else int(stream_nt)
         self.shape_from_ref = bool(shape_from_ref)
         p.shape_from_ref = 1 if shape_from_ref else 0
-        p.scatter = _lib.SCATTER_TILED
+        p.scatter, p.tile_odd = _lib.SCATTER_TILED, 1
         p.tile_k, p.tile_max_nodes = K, MX
         p.tile_count, p.tile_nodes, p.tile_lend = (t.data_ptr() for t in (self.t_count, self.t_nodes, self.t_lend))
         p.tile_corners, p.tile_dst = self.t_corners.data_ptr(), self.t_dst.data_ptr()

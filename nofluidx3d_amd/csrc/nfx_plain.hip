@@ -466,7 +466,11 @@ __device__ __forceinline__ void node_step(const NodeStep& s, const float* __rest
 // with, for each, the end of its run in the tile's corner list sorted by (node, slot) (tile_lend)
 // and the position of its partial sum in node order (tile_dst).  Each corner slot 4*(t-t0)+a
 // carries its tile-local node and its rank in that node's run (tile_corners), so its place in the
-// sorted list is run start + rank.  Phases:
+// sorted list is run start + rank.  Where tiles do not carry node updates their nodes are in the order of
+// their run length and run starts lie at odd distances (nfx_order_tiles_host, a.odd): the threads that sum
+// runs of one length then read different LDS banks at every step (2.65 M tetra cell: bank conflicts 6.5 M -> 4.3 M
+// of 12.1 M -> 9.6 M LDS cycles per launch, step -2 to -3 %).  A node-fused launch also gathers and stores its
+// nodes and lost 1.6 % to the order: its lists keep ascending ids.  Phases:
 //   0  issue the tetra's streaming loads (Dm^-1 and V0 unless GEO, the viscoplastic state and epsbar),
 //      its corner records and the tile metadata
 //   1  node displacements (GEO: and reference positions) and run starts -> LDS
@@ -493,6 +497,7 @@ struct TileArgs {
     const uint32_t* __restrict__ tile_dst;
     float* __restrict__ partials;
     int32_t max_nodes;
+    int32_t odd;  // 1: run starts at odd distances
     // viscoplastic, nullable: per tile, 0 = every tetra of the tile has a zero plastic state (its
     // state is neither read nor written until one of them flows; the tile then sets its flag)
     uint32_t* __restrict__ vp_active;
@@ -555,13 +560,13 @@ __device__ void batch_curve_sample(const float* __restrict__ x, const float* __r
     }
 }
 
-// LDS of a tile: corner forces 12K floats, then per tile-node its displacement and X0.x (16 B), with
-// GEO X0.y and X0.z (8 B), and its run start (u16)
-template <int K>
-__host__ __device__ constexpr size_t tile_lds_bytes_fixed() {
-    return 4 * 12 * K;
+// LDS of a tile: three components of the corner list (4K corners and, for odd run distances, a pad per
+// tile-node at most), then per tile-node its displacement and X0.x (16 B), with GEO X0.y and X0.z (8 B),
+// and its run start (u16)
+__host__ __device__ constexpr int tile_corner_slots(int K, bool node) { return 4 * K + (node ? 0 : K < 256 ? K : 256); }
+__host__ __device__ constexpr size_t tile_lds_bytes(int K, int max_nodes, bool geo, bool node) {
+    return (size_t)12 * tile_corner_slots(K, node) + (size_t)(16 + (geo ? 8 : 0) + 2) * max_nodes;
 }
-__host__ __device__ constexpr size_t tile_lds_bytes_per_node(bool geo) { return 16 + (geo ? 8 : 0) + 2; }
 
 // GEO: Dm^-1 and V0 from the staged reference positions; NT: cache policy of the streams; EPS: the
 // viscoplastic law keeps its accumulated plastic strain (the linear law does not read it); SYM: its
@@ -577,11 +582,12 @@ __global__ __launch_bounds__(K, MODEL != NFX_VISCOPLASTIC ? 8 : (STRESS || NODE)
                                                   float* __restrict__ pr) {
     // one thread per tetra of the tile (blockDim.x == K)
     extern __shared__ __align__(16) unsigned char smem[];
-    float* s_cf = reinterpret_cast<float*>(smem);  // [component][4K], sorted-corner order
+    constexpr int CS = tile_corner_slots(K, NODE);
+    float* s_cf = reinterpret_cast<float*>(smem);  // [component][CS], sorted-corner order
     const int MX = a.max_nodes;
     // per tile-node, node-major: (ux, uy, uz, X0x) as one 16-byte LDS word and, with GEO, (X0y, X0z)
     // as one 8-byte word, so a corner's node data is one or two LDS reads at one address
-    float4* s_n = reinterpret_cast<float4*>(s_cf + 12 * K);
+    float4* s_n = reinterpret_cast<float4*>(s_cf + 3 * CS);
     __shared__ int s_flow;                         // viscoplastic: a tetra of the tile flowed this step
     __shared__ double s_tip[NODE ? K / 64 : 1];    // NODE: per wave, the indenter force of the previous step
     float2* s_r = reinterpret_cast<float2*>(s_n + MX);
@@ -660,6 +666,7 @@ __global__ __launch_bounds__(K, MODEL != NFX_VISCOPLASTIC ? 8 : (STRESS || NODE)
             dst = ld_g<NT, uint32_t>(uat(a.tile_dst + j0, u));
         }
         lb = tl ? ld_g<NT, uint16_t>(uat(a.tile_lend + j0, u - 1)) : 0;
+        if constexpr (!NODE) lb += (lb ^ tl) & a.odd;  // the first place of the run's parity
         le = ld_g<NT, uint16_t>(uat(a.tile_lend + j0, u));
     }
     // this tetra's 4 corner records (tile-node | rank << 8), as one 8-byte load
@@ -771,13 +778,13 @@ __global__ __launch_bounds__(K, MODEL != NFX_VISCOPLASTIC ? 8 : (STRESS || NODE)
         } else {
             f = svkk_tetra(H, D, vs, e.mu, e.kappa_svk);
         }
-        // each corner's place in the tile's (node, slot)-sorted corner list: run start + rank
+        // each corner's place in the tile's corner list: run start + rank
         const int q0 = s_lb[l0] + (int)((cr >> 8) & 0xFF), q1 = s_lb[l1] + (int)((cr >> 24) & 0xFF);
         const int q2 = s_lb[l2] + (int)((cr >> 40) & 0xFF), q3 = s_lb[l3] + (int)((cr >> 56) & 0xFF);
-        s_cf[q0] = f.f0.x; s_cf[4 * K + q0] = f.f0.y; s_cf[8 * K + q0] = f.f0.z;
-        s_cf[q1] = f.f1.x; s_cf[4 * K + q1] = f.f1.y; s_cf[8 * K + q1] = f.f1.z;
-        s_cf[q2] = f.f2.x; s_cf[4 * K + q2] = f.f2.y; s_cf[8 * K + q2] = f.f2.z;
-        s_cf[q3] = f.f3.x; s_cf[4 * K + q3] = f.f3.y; s_cf[8 * K + q3] = f.f3.z;
+        s_cf[q0] = f.f0.x; s_cf[CS + q0] = f.f0.y; s_cf[2 * CS + q0] = f.f0.z;
+        s_cf[q1] = f.f1.x; s_cf[CS + q1] = f.f1.y; s_cf[2 * CS + q1] = f.f1.z;
+        s_cf[q2] = f.f2.x; s_cf[CS + q2] = f.f2.y; s_cf[2 * CS + q2] = f.f2.z;
+        s_cf[q3] = f.f3.x; s_cf[CS + q3] = f.f3.y; s_cf[2 * CS + q3] = f.f3.z;
     }
     if (MODEL == NFX_VISCOPLASTIC && flows) s_flow = 1;  // any flowing lane; all write the same value
     __syncthreads();
@@ -789,14 +796,14 @@ __global__ __launch_bounds__(K, MODEL != NFX_VISCOPLASTIC ? 8 : (STRESS || NODE)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 fx += s_cf[q + i];
-                fy += s_cf[4 * K + q + i];
-                fz += s_cf[8 * K + q + i];
+                fy += s_cf[CS + q + i];
+                fz += s_cf[2 * CS + q + i];
             }
         }
         for (; q < le; ++q) {
             fx += s_cf[q];
-            fy += s_cf[4 * K + q];
-            fz += s_cf[8 * K + q];
+            fy += s_cf[CS + q];
+            fz += s_cf[2 * CS + q];
         }
         float* o = a.partials + 3 * (int64_t)dst;
         o[0] = fx;
@@ -1162,7 +1169,7 @@ static int validate_plan(const nfx_plan* p) {
         NFX_REQUIRE(p->tile_max_nodes > 0 && p->tile_max_nodes <= p->tile_k && p->tile_max_nodes <= 256,
                     "plan: tile_max_nodes %d exceeds tile_k %d or 256 (use another tile size or scatter mode)",
                     p->tile_max_nodes, p->tile_k);
-        const size_t lds = (size_t)p->tile_k * 48 + tile_lds_bytes_per_node(p->shape_from_ref != 0) * (size_t)p->tile_max_nodes;
+        const size_t lds = tile_lds_bytes(p->tile_k, p->tile_max_nodes, p->shape_from_ref != 0, false);
         NFX_REQUIRE(lds <= 65536, "plan: tile needs %zu B of LDS (max 65536); use a smaller tile_k", lds);
     }
     NFX_REQUIRE(p->scatter != NFX_SCATTER_ATOMIC || p->force, "plan: atomic scatter needs force");
@@ -1175,6 +1182,7 @@ static int validate_plan(const nfx_plan* p) {
                 "plan: the node-fused arrays disp_b, vel_b, partials_b and tile_range are set together");
     NFX_REQUIRE(nb == 0 || (p->scatter == NFX_SCATTER_TILED && p->model >= NFX_SVKK && p->model <= NFX_VISCOPLASTIC),
                 "plan: node-fused steps need the tiled scatter and model NFX_SVKK, NFX_SVK, NFX_MR or NFX_VISCOPLASTIC");
+    NFX_REQUIRE(nb == 0 || !p->tile_odd, "plan: node-fused steps take the tile arrays as nfx_build_tiles_host filled them");
     NFX_REQUIRE(nb == 0 || (p->disp_b != p->disp && p->vel_b != p->vel && p->partials_b != p->partials),
                 "plan: the node-fused buffers must differ from disp, vel and partials");
     return NFX_OK;
@@ -1243,7 +1251,7 @@ static void launch_tiled_k(nfx_ctx* ctx, const nfx_plan& p, bool st, const Fused
     // ctx->batch is set only while a batched step is being enqueued
     TileArgs a{p.N,          p.T,         p.dminv,        p.v0,       p.disp,     p.ref,
                p.tile_count, p.tile_nodes, p.tile_lend,    p.tile_corners, p.tile_dst, p.partials,
-               p.tile_max_nodes};
+               p.tile_max_nodes, p.tile_odd != 0};
     if (p.model == NFX_VISCOPLASTIC) a.vp_active = p.vp_active;
     if constexpr (NODE) {
         a.x = io->x;
@@ -1294,7 +1302,7 @@ static void launch_tiled_k(nfx_ctx* ctx, const nfx_plan& p, bool st, const Fused
         }
     }
     const unsigned int nb = (unsigned int)((p.T + K - 1) / K) + (unsigned int)a.curve_blocks;
-    const size_t lds = tile_lds_bytes_fixed<K>() + tile_lds_bytes_per_node(GEO) * (size_t)p.tile_max_nodes;
+    const size_t lds = tile_lds_bytes(K, p.tile_max_nodes, GEO, NODE);
     const ElasticDev e = elastic_consts(p);
     const VPConst c = vp_consts(p.vp);
     hipStream_t s = ctx->stream;
@@ -2144,6 +2152,43 @@ int nfx_build_tiles_host(const uint32_t* tet, int64_t N, int64_t T, int32_t K, i
     std::memcpy(node_off, cnt.data(), sizeof(uint32_t) * (size_t)(N + 1));
     for (int64_t c = 0; c < ntiles; ++c)
         for (uint32_t i = 0; i < tile_count[c]; ++i) tile_dst[c * MX + i] = cnt[tile_nodes[c * MX + i]]++;
+    return NFX_OK;
+}
+
+int nfx_order_tiles_host(int64_t ntiles, int32_t K, int32_t MX, const uint32_t* tile_count, uint32_t* tile_nodes,
+                         uint16_t* tile_lend, uint16_t* tile_corners, uint32_t* tile_dst, uint16_t* perm) {
+    NFX_REQUIRE(tile_count && tile_nodes && tile_lend && tile_corners && tile_dst && perm, "NULL argument");
+    NFX_REQUIRE(ntiles > 0 && (K == 128 || K == 256 || K == 512) && MX > 0 && MX <= 256 && MX <= K, "bad tile shape");
+    uint32_t nodes[256], dst[256];
+    uint16_t at[256];
+    int len[256];
+    for (int64_t c = 0; c < ntiles; ++c) {
+        const int M = (int)tile_count[c];
+        NFX_REQUIRE(M > 0 && M <= MX, "tile %lld: %d tile-nodes outside 1..%d", (long long)c, M, MX);
+        uint16_t* lend = tile_lend + c * MX;
+        const int total = lend[M - 1];
+        for (int j = 0; j < M; ++j) {
+            len[j] = (int)lend[j] - (j ? (int)lend[j - 1] : 0);
+            NFX_REQUIRE(len[j] > 0 && total <= 4 * K, "tile %lld: bad run ends", (long long)c);
+        }
+        uint16_t* q = tile_corners + (size_t)4 * K * c;
+        for (int i = 0; i < total; ++i)
+            NFX_REQUIRE((q[i] & 0xFF) < M, "tile %lld: corner of tile-node %d", (long long)c, q[i] & 0xFF);
+        uint16_t* p = perm + c * MX;
+        for (int j = 0; j < MX; ++j) p[j] = (uint16_t)j;
+        std::stable_sort(p, p + M, [&](uint16_t a, uint16_t b) { return len[a] > len[b]; });
+        int start = 0;
+        for (int j = 0; j < M; ++j) {
+            nodes[j] = tile_nodes[c * MX + p[j]];
+            dst[j] = tile_dst[c * MX + p[j]];
+            lend[j] = (uint16_t)(start + len[p[j]]);
+            start += len[p[j]] | 1;
+            at[p[j]] = (uint16_t)j;
+        }
+        std::copy(nodes, nodes + M, tile_nodes + c * MX);
+        std::copy(dst, dst + M, tile_dst + c * MX);
+        for (int i = 0; i < total; ++i) q[i] = (uint16_t)((q[i] & 0xFF00) | at[q[i] & 0xFF]);
+    }
     return NFX_OK;
 }
 
