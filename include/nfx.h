@@ -58,6 +58,9 @@ extern "C" {
 
 typedef struct nfx_ctx nfx_ctx;
 
+/* nfx_init's stream argument for the device's default (null) stream */
+#define NFX_STREAM_DEFAULT ((void*)1)
+
 /* Elastic constants in simulation units: the #defines of interactions/Tetra.py:66-79, and the
  * per-tetra parameter arrays of the legacy laws (uniform here). */
 typedef struct {
@@ -210,8 +213,8 @@ typedef struct {
 /* ---- device and queue: replaces openCL.py:17-50 -------------------------------------------- */
 int nfx_device_count(int* count);                        /* openCL.py:20-28 device walk */
 int nfx_init(int device_id, void* stream, nfx_ctx** ctx); /* openCL.py:17-34 initializeOpenCLObjects;
-                                                             stream: hipStream_t to use, or NULL for a
-                                                             library-owned default-priority stream */
+                                                             stream: hipStream_t to use, NFX_STREAM_DEFAULT, or
+                                                             NULL for a library-owned default-priority stream */
 int nfx_destroy(nfx_ctx* ctx);
 int nfx_stream_sync(nfx_ctx* ctx); /* getCommandQueue().finish(), Simulation.py:266 */
 const char* nfx_last_error(void);

@@ -16,6 +16,8 @@ NFX_SVKK, NFX_SVK, NFX_MR, NFX_VISCOPLASTIC = 0, 1, 2, 3
 NFX_LINEAR_ELASTIC, NFX_LINEAR_DEVIATORIC, NFX_NEO_HOOKEAN_2, NFX_PORO_NEO_HOOKEAN = 4, 5, 6, 7
 SCATTER_ATOMIC, SCATTER_CSR, SCATTER_TILED = 0, 1, 2
 INDENTER_NONE, INDENTER_SPHERE, INDENTER_PLANE = 0, 1, 2
+# nfx_init: the device's default (null) stream
+STREAM_DEFAULT = 1
 
 c_i32, c_i64, c_f64, c_vp = ctypes.c_int32, ctypes.c_int64, ctypes.c_double, ctypes.c_void_p
 

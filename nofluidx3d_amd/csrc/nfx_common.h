@@ -54,6 +54,7 @@ struct nfx_ctx {
     int num_cu = 0;
     hipStream_t stream = nullptr;
     bool own_stream = false;
+    hipStream_t capture = nullptr;  // records step blocks when stream is the default stream, which cannot
     double* partials = nullptr;       // kMaxReduceBlocks * 2 doubles
     unsigned int* counter = nullptr;  // 1 counter (reset by the last block of each reduction)
     int64_t* step_dev = nullptr;      // device step counter for graph replays

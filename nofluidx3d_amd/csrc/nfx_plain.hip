@@ -1677,7 +1677,14 @@ static int capture_graph(nfx_ctx* ctx, const nfx_plan& p, const nfx_batch* b, bo
         if (ctx->graphs[old].graph) (void)hipGraphDestroy(ctx->graphs[old].graph);
         ctx->graphs.erase(ctx->graphs.begin() + (std::ptrdiff_t)old);
     }
-    NFX_HIP(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeGlobal));
+    const hipStream_t run = ctx->stream;
+    if (ctx->capture) ctx->stream = ctx->capture;
+    const hipError_t eb = hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeGlobal);
+    if (eb != hipSuccess) {
+        ctx->stream = run;
+        set_error("hipStreamBeginCapture failed: %s", hipGetErrorString(eb));
+        return NFX_ERR_HIP;
+    }
     int rc = NFX_OK;
     for (int64_t i = 0; i < kGraphBlock && rc == NFX_OK; ++i) {
         if (b) {
@@ -1705,6 +1712,7 @@ static int capture_graph(nfx_ctx* ctx, const nfx_plan& p, const nfx_batch* b, bo
     }
     hipGraph_t g = nullptr;
     const hipError_t e = hipStreamEndCapture(ctx->stream, &g);
+    ctx->stream = run;
     if (rc != NFX_OK) {
         if (g) (void)hipGraphDestroy(g);
         return rc;
@@ -1826,7 +1834,9 @@ static int init_ctx(nfx_ctx* c, void* stream) {
     hipDeviceProp_t prop;
     NFX_HIP(hipGetDeviceProperties(&prop, c->device));
     c->num_cu = prop.multiProcessorCount;
-    if (stream) {
+    if (stream == NFX_STREAM_DEFAULT) {
+        NFX_HIP(hipStreamCreateWithFlags(&c->capture, hipStreamNonBlocking));
+    } else if (stream) {
         c->stream = (hipStream_t)stream;
     } else {
         NFX_HIP(hipStreamCreate(&c->stream));
@@ -1881,6 +1891,7 @@ int nfx_destroy(nfx_ctx* c) {
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     if (c->own_stream) (void)hipStreamDestroy(c->stream);
+    if (c->capture) (void)hipStreamDestroy(c->capture);
     delete c;
     return NFX_OK;
 }

@@ -1,7 +1,7 @@
 """Device, context and queue singletons (the API of reference ``nofluidx3d/openCL.py:17-50``).
 
 ``initializeOpenCLObjects(deviceId)`` selects HIP device ``deviceId`` and creates the libnfx
-context with its own default-priority stream; ``getCommandQueue().finish()`` waits for it.  As
+context on the device's default stream; ``getCommandQueue().finish()`` waits for it.  As
 in the reference, a missing device id prints an error and exits with status 1
 (``openCL.py:30-32``).
 """
@@ -32,7 +32,11 @@ class Context:
         self.torch_device = torch.device("cuda", device_id)
         torch.cuda.set_device(device_id)
         h = ctypes.c_void_p()
-        _lib.call("nfx_init", device_id, None, ctypes.byref(h))
+        # torch's default stream: device work of torch and of the library is in one queue, in order.  A
+        # stream of the library's own would be ordered with it too, but by waits on both sides for every
+        # torch operation between two calls (measured: a training step of the surrogate 524 us so, 347 us
+        # on the default stream; 1000 steps with a torch operation after them 9.2 and 6.9 ms)
+        _lib.call("nfx_init", device_id, _lib.STREAM_DEFAULT, ctypes.byref(h))
         self.handle = h.value
         buf = ctypes.create_string_buffer(256)
         _lib.call("nfx_device_name", self.handle, buf, 256)
