@@ -257,10 +257,11 @@ struct LveConst {
 };
 
 template <bool CORNERS>
-__global__ __launch_bounds__(kB) void k_lve(float* f, float* corners, const float* __restrict__ x,
-                                            const uint32_t* __restrict__ tets, const float* __restrict__ dminv,
-                                            int64_t N, int64_t T, LveConst c, float* dev_old, float* transient,
-                                            float* vm, float* pr) {
+__global__ __launch_bounds__(kB) void k_lve(float* __restrict__ f, float* __restrict__ corners,
+                                            const float* __restrict__ x, const uint32_t* __restrict__ tets,
+                                            const float* __restrict__ dminv, int64_t N, int64_t T, LveConst c,
+                                            float* __restrict__ dev_old, float* __restrict__ transient,
+                                            float* __restrict__ vm, float* __restrict__ pr) {
     const int64_t t = (int64_t)blockIdx.x * kB + threadIdx.x;
     if (t >= T) return;
     const uint32_t n0 = tets[t], n1 = tets[T + t], n2 = tets[2 * T + t], n3 = tets[3 * T + t];
@@ -275,24 +276,45 @@ __global__ __launch_bounds__(kB) void k_lve(float* f, float* corners, const floa
 #pragma unroll
         for (int k = 0; k < 3; ++k) e[i][k] = 0.5f * (F.m[i][k] + F.m[k][i]) - (i == k ? 1.0f : 0.0f);
     const float tr = e[0][0] + e[1][1] + e[2][2];
-    float sig[3][3];
+    // the state in planes of nine entries, each plane's loads together and the next term's issued before this
+    // one is stored: nterms + 1 memory rounds in flight instead of 9 (nterms + 1) one after another
+    float old[9], h[9], rate[9], sig[3][3], t3;
+    {
+#pragma clang fp contract(off)
+        t3 = tr * (1.0f / 3.0f);
+    }
+#pragma unroll
+    for (int q = 0; q < 9; ++q) old[q] = dev_old[q * T + t];
+    if (c.nterms) {
+#pragma unroll
+        for (int q = 0; q < 9; ++q) h[q] = transient[q * T + t];
+    }
 #pragma unroll
     for (int i = 0; i < 3; ++i)
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
             const int q = 3 * i + k;
-            const float dv = e[i][k] - (i == k ? tr * (1.0f / 3.0f) : 0.0f);
-            const float rate = dv - dev_old[q * T + t];
+            // the trace's third is rounded on its own but in the first entry: the results of the form with one
+            // loop over the terms per entry, bit for bit
+            const float dv = i != k ? e[i][k] : i == 0 ? __builtin_fmaf(tr, -1.0f / 3.0f, e[i][k]) : e[i][k] - t3;
+            rate[q] = dv - old[q];
             dev_old[q * T + t] = dv;
-            float s = c.two_mu_inf * dv + (i == k ? c.kappa * tr : 0.0f);
-            for (int j = 0; j < c.nterms; ++j) {
-                float* h = &transient[(9 * (int64_t)j + q) * T + t];
-                const float hn = c.decay[j] * *h + c.two_mu * c.w[j] * rate;
-                *h = hn;
-                s += hn;
-            }
-            sig[i][k] = s;
+            sig[i][k] = c.two_mu_inf * dv + (i == k ? c.kappa * tr : 0.0f);
         }
+    for (int j = 0; j < c.nterms; ++j) {
+        float next[9];
+        if (j + 1 < c.nterms) {
+#pragma unroll
+            for (int q = 0; q < 9; ++q) next[q] = transient[(9 * (int64_t)(j + 1) + q) * T + t];
+        }
+#pragma unroll
+        for (int q = 0; q < 9; ++q) {
+            const float hn = c.decay[j] * h[q] + c.two_mu * c.w[j] * rate[q];
+            transient[(9 * (int64_t)j + q) * T + t] = hn;
+            sig[q / 3][q % 3] += hn;
+            h[q] = next[q];
+        }
+    }
     // the legacy kernel keeps sigma as computed (symmetric up to rounding); its face forces use the rows
     const S6 S{sig[0][0], sig[1][1], sig[2][2], 0.5f * (sig[0][1] + sig[1][0]), 0.5f * (sig[1][2] + sig[2][1]),
                0.5f * (sig[0][2] + sig[2][0])};

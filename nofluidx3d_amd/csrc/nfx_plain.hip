@@ -916,10 +916,20 @@ template <int G>
 __device__ __forceinline__ V3 gather_node(const NodeArgs& a, int64_t n, int sub) {
     V3 f = mk(0.f, 0.f, 0.f);
     const uint32_t b = a.off[n], e = a.off[n + 1];
-    for (uint32_t j = b + sub; j < e; j += G) {
-        const uint32_t s = a.slots[j];
-        const float* p = a.corners + 12 * (int64_t)(s >> 2) + 3 * (s & 3);
-        f = f + mk(p[0], p[1], p[2]);
+    // eight slots' loads, then their records' loads together: two memory rounds for nodes of up to 8 G corners
+    // instead of two per G corners (the last ones repeat the lane's first slot and count zero; same sums)
+    for (uint32_t j = b + sub; j < e; j += 8 * G) {
+        uint32_t s[8];
+        V3 q[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) s[i] = a.slots[j + i * G < e ? j + i * G : j];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float* p = a.corners + 12 * (int64_t)(s[i] >> 2) + 3 * (s[i] & 3);
+            q[i] = mk(p[0], p[1], p[2]);
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) f = f + (j + i * G < e ? q[i] : mk(0.f, 0.f, 0.f));
     }
 #pragma unroll
     for (int o = 1; o < G; o <<= 1) {
