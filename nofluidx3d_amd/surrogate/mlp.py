@@ -32,9 +32,9 @@ def _pad32(n):
 
 
 def split_k(M, N, K, min_groups=512, max_split=64):
-    """K slices for a GEMM of M x N outputs over K: doubled until the grid has ``min_groups``
-    workgroups of 128 x 32 outputs (the weight-gradient GEMMs have few outputs and K = batch),
-    each slice a multiple of 32 long"""
+    """K slices for a GEMM of M x N outputs over K: doubled until there are ``min_groups`` tiles of
+    128 x 32 outputs, each the work of two workgroups (the weight-gradient GEMMs have few outputs
+    and K = batch), each slice a multiple of 32 long"""
     groups = (M // 128) * (N // 32)
     s = 1
     while s < max_split and groups * s < min_groups and K % (64 * s) == 0:
