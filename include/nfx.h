@@ -383,8 +383,9 @@ int nfx_graph_captures(nfx_ctx* ctx, int64_t* count);
 int nfx_node_update(nfx_ctx* ctx, const nfx_plan* plan, int64_t step, double* tip_out);
 
 /* ---- batched stepping (no reference counterpart; the reference simulates one cell per process):
- *      all cells of the batch advance together, one force pass + one node pass per step over the
- *      concatenated meshes, plus a per-cell curve-sampling pass; plan holds the concatenated mesh,
+ *      all cells of the batch advance together, one force pass (which also samples the curves) + one node pass
+ *      per step over the concatenated meshes; with the node-fused buffers in the plan, one launch per step as in
+ *      nfx_run_steps (same bits; a batch keeps w in vel between calls); plan holds the concatenated mesh,
  *      state and tile arrays (scatter must be NFX_SCATTER_TILED, model NFX_MR or NFX_VISCOPLASTIC,
  *      the substrate/indenter flags select the terms; their values come from the cell table). ---- */
 int nfx_batch_run_steps(nfx_ctx* ctx, const nfx_plan* plan, const nfx_batch* batch, int64_t step0, int64_t nsteps,

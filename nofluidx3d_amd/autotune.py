@@ -47,12 +47,14 @@ def default_stream_nt(tetra):
 # millions of tetra its force pass, which then also updates every node it touches (~2.9 times per
 # node), is longer than the two passes apart.  Measured on MI355X (NH cells, best tile shape of each
 # form, us per graph-replayed step, fused against two launches): 25k tetra 5.5 / 7.2, 106k 6.3 / 7.9,
-# 211k 7.5 / 8.8, 526k 11.7 / 12.5, 878k 16.6 / 16.5; the 3.4M-tetra viscoplastic cell 58 / 50
+# 211k 7.5 / 8.8, 526k 11.7 / 12.5, 878k 16.6 / 16.5; the 3.4M-tetra viscoplastic cell 58 / 50.  Batches,
+# curve samples in the launch (elastic, viscoplastic): 46k 6.2 / 8.2, 6.3 / 8.9; 234k 8.1 / 10.0, 9.2 / 11.5; 780k
+# 15.4 / 15.5, 21.7 / 22.7
 NODE_FUSED_MAX_TETRA = 600_000
 
 
 def default_node_fused(tetra):
-    """the step form to use untuned: node-fused for meshes of at most NODE_FUSED_MAX_TETRA tetra"""
+    """the step form of a mesh or batch to use untuned: node-fused for at most NODE_FUSED_MAX_TETRA tetra"""
     return int(tetra) <= NODE_FUSED_MAX_TETRA
 
 

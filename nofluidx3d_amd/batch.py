@@ -31,8 +31,8 @@ import os
 import numpy as np
 
 from nofluidx3d_amd import _lib
-from nofluidx3d_amd.autotune import default_stream_nt
-from nofluidx3d_amd.Simulation import order_tiles
+from nofluidx3d_amd.autotune import default_node_fused, default_stream_nt
+from nofluidx3d_amd.Simulation import order_tiles, tile_ranges
 
 E_SIM = 1e-2
 
@@ -344,6 +344,7 @@ class BatchSimulation:
     Q = Fp^-1 - I (9);
     ``narrow`` 16-bit tile-node ids and partial positions (when every cell has < 65536 nodes);
     ``shape_from_ref`` the force pass forms Dm^-1 from the reference positions instead of streaming it.
+    Batches of at most ``autotune.NODE_FUSED_MAX_TETRA`` tetra run the node-fused step (same bits).
 
     State on the device: node displacements u from the FP32 reference positions X0 (``ref``), the
     velocity-Verlet state w = a v + f/2, and for the viscoplastic law the plastic deviation Gd
@@ -369,7 +370,10 @@ class BatchSimulation:
             raise ValueError("a batch is either all elastic or all viscoplastic")
         self.model = _lib.NFX_VISCOPLASTIC if viscous[0] else _lib.NFX_MR
         h = build_host_arrays(specs, meshes, steps, K)
-        order_batch_tiles(h, K)
+        # one launch per step where launches dominate it, as for single cells (every node a corner of some tetra)
+        fuse = default_node_fused(h["T_real"]) and bool((np.diff(h["node_poff"].astype(np.int64)) > 0).all())
+        if not fuse:
+            order_batch_tiles(h, K)
         self._meshes = meshes
         self.cells_host, self.units, self.radius_sim = h["cells"], h["units"], h["radius_sim"]
         self.node_off, self.tet_pad_off = h["node_off"], h["tet_pad_off"]
@@ -446,12 +450,18 @@ class BatchSimulation:
         p.stream_nt = default_stream_nt(self.T) if stream_nt is None else int(stream_nt)
         self.shape_from_ref = bool(shape_from_ref)
         p.shape_from_ref = 1 if shape_from_ref else 0
-        p.scatter, p.tile_odd = _lib.SCATTER_TILED, 1
+        p.scatter, p.tile_odd = _lib.SCATTER_TILED, 0 if fuse else 1
         p.tile_k, p.tile_max_nodes = K, MX
         p.tile_count, p.tile_nodes, p.tile_lend = (t.data_ptr() for t in (self.t_count, self.t_nodes, self.t_lend))
         p.tile_corners, p.tile_dst = self.t_corners.data_ptr(), self.t_dst.data_ptr()
         p.node_off, p.partials = self.node_poff.data_ptr(), self.partials.data_ptr()
         p.substrate, p.indenter = 1, _lib.INDENTER_SPHERE
+        if fuse:
+            self.t_range = u32(tile_ranges(h["tile_nodes"], h["tile_count"], h["node_poff"], MX))
+            self.x_b, self.v_b, self.partials_b = (torch.zeros_like(t) for t in (self.x, self.v, self.partials))
+            torch.cuda.synchronize(dev)
+            p.disp_b, p.vel_b, p.partials_b = self.x_b.data_ptr(), self.v_b.data_ptr(), self.partials_b.data_ptr()
+            p.tile_range = self.t_range.data_ptr()
         self.plan = p
         b = Batch()
         b.ncells = nc

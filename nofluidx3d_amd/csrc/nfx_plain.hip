@@ -403,6 +403,11 @@ __device__ __forceinline__ void node_contacts(const float* __restrict__ ref, int
     }
 }
 
+// the constants of a cell's contacts
+struct ContactConsts {
+    double sub_k, wall, ind_k, ind_radius, ind_start, ind_speed, ind_move;
+};
+
 // The previous step's node update riding in a node-fused force pass: every tile that touches node n
 // updates it from the same inputs with the same operations (so the copies agree bitwise) and the
 // node's first tile (its partial is the node's first, dst == node_off[n]) stores the result.
@@ -415,7 +420,7 @@ struct NodeStep {
     float* __restrict__ w_next;
     double* __restrict__ tip_row;  // nullable: per tile, the indenter force on the nodes it stores
     int32_t substrate, indenter, fix, vv_first;
-    double sub_k, wall, ind_k, ind_radius, ind_start, ind_speed, ind_move;
+    ContactConsts cc;  // batches take each tile's from its cell instead
     int64_t step;  // the step being completed (step_dev + step_off when step_dev is set)
     const int64_t* step_dev;
     int32_t step_off;
@@ -424,23 +429,24 @@ struct NodeStep {
 // node n's update (k_node_update's arithmetic, the substrate/indenter/fix choices uniform at run
 // time): x holds u before the step on entry and after it on return; tip receives the node's indenter
 // force when this tile stores the node
-__device__ __forceinline__ void node_step(const NodeStep& s, const float* __restrict__ ref, int64_t N, uint32_t n,
-                                          uint32_t dst, uint2 rg, double pos, V3& x, double& tip) {
+__device__ __forceinline__ void node_step(const NodeStep& s, const ContactConsts& cc, const float* __restrict__ ref,
+                                          int64_t N, uint32_t n, uint32_t dst, uint2 rg, double pos, V3& x,
+                                          double& tip) {
     const uint32_t b = rg.x, e = rg.y;
     V3 f = sum_partials8(s.prev_partials, b, e);
     double tf = 0.0, td = 0.0;
     if (s.substrate) {
         if (s.indenter == NFX_INDENTER_SPHERE)
-            node_contacts<true, NFX_INDENTER_SPHERE>(ref, N, n, x, s.sub_k, s.wall, s.ind_k, s.ind_radius, pos, f, tf, td);
+            node_contacts<true, NFX_INDENTER_SPHERE>(ref, N, n, x, cc.sub_k, cc.wall, cc.ind_k, cc.ind_radius, pos, f, tf, td);
         else if (s.indenter == NFX_INDENTER_PLANE)
-            node_contacts<true, NFX_INDENTER_PLANE>(ref, N, n, x, s.sub_k, s.wall, s.ind_k, s.ind_radius, pos, f, tf, td);
+            node_contacts<true, NFX_INDENTER_PLANE>(ref, N, n, x, cc.sub_k, cc.wall, cc.ind_k, cc.ind_radius, pos, f, tf, td);
         else
-            node_contacts<true, NFX_INDENTER_NONE>(ref, N, n, x, s.sub_k, s.wall, s.ind_k, s.ind_radius, pos, f, tf, td);
+            node_contacts<true, NFX_INDENTER_NONE>(ref, N, n, x, cc.sub_k, cc.wall, cc.ind_k, cc.ind_radius, pos, f, tf, td);
     } else {
         if (s.indenter == NFX_INDENTER_SPHERE)
-            node_contacts<false, NFX_INDENTER_SPHERE>(ref, N, n, x, s.sub_k, s.wall, s.ind_k, s.ind_radius, pos, f, tf, td);
+            node_contacts<false, NFX_INDENTER_SPHERE>(ref, N, n, x, cc.sub_k, cc.wall, cc.ind_k, cc.ind_radius, pos, f, tf, td);
         else if (s.indenter == NFX_INDENTER_PLANE)
-            node_contacts<false, NFX_INDENTER_PLANE>(ref, N, n, x, s.sub_k, s.wall, s.ind_k, s.ind_radius, pos, f, tf, td);
+            node_contacts<false, NFX_INDENTER_PLANE>(ref, N, n, x, cc.sub_k, cc.wall, cc.ind_k, cc.ind_radius, pos, f, tf, td);
     }
     V3 w = mk(s.w[n], s.w[N + n], s.w[2 * N + n]);
     if (s.vv_first) {
@@ -623,9 +629,12 @@ __global__ __launch_bounds__(K, MODEL != NFX_VISCOPLASTIC ? 8 : (STRESS || NODE)
     const int64_t T = a.T, N = a.N;
     const int64_t t0 = c * K;
     int nt = (int)((T - t0) < K ? (T - t0) : K);
+    ContactConsts cc = a.ns.cc;  // NODE
     if (a.cells) {  // batch: this tile's cell and its constants (uniform over the workgroup)
         nt = a.tile_ntet[c];
         const nfx_cell cp = a.cells[a.tile_cell[c]];
+        if constexpr (NODE)
+            cc = {cp.substrate_k, cp.wall, cp.tip_k, cp.tip_radius, cp.tip_start, cp.tip_speed, cp.tip_move_steps};
         e.mu1 = cp.mu1;
         e.mu2 = cp.mu2;
         e.kappa = cp.kappa;
@@ -699,10 +708,10 @@ __global__ __launch_bounds__(K, MODEL != NFX_VISCOPLASTIC ? 8 : (STRESS || NODE)
             double pos = 0.0;
             if (a.ns.indenter) {
                 const int64_t time = a.ns.step_dev ? (*a.ns.step_dev + a.ns.step_off) : a.ns.step;
-                pos = indenter_pos(a.ns.ind_start, a.ns.ind_speed, a.ns.ind_move, time);
+                pos = indenter_pos(cc.ind_start, cc.ind_speed, cc.ind_move, time);
             }
             V3 xn = mk(ux, uy, uz);
-            node_step(a.ns, a.ref, N, nid, dst, rg, pos, xn, tip);
+            node_step(a.ns, cc, a.ref, N, nid, dst, rg, pos, xn, tip);
             ux = xn.x;
             uy = xn.y;
             uz = xn.z;
@@ -1295,15 +1304,9 @@ static void launch_tiled_k(nfx_ctx* ctx, const nfx_plan& p, bool st, const Fused
         n.tip_row = io->tip_row;
         n.substrate = p.substrate;
         n.indenter = p.indenter;
-        n.fix = p.fix_top_bottom;
+        n.fix = ctx->batch ? 0 : p.fix_top_bottom;  // as k_batch_node
         n.vv_first = io->vv_first;
-        n.sub_k = p.substrate_k;
-        n.wall = p.wall;
-        n.ind_k = p.ind_k;
-        n.ind_radius = p.ind_radius;
-        n.ind_start = p.ind_start;
-        n.ind_speed = p.ind_speed;
-        n.ind_move = p.ind_move_steps;
+        n.cc = {p.substrate_k, p.wall, p.ind_k, p.ind_radius, p.ind_start, p.ind_speed, p.ind_move_steps};
         n.step = io->step;
         n.step_dev = io->step_dev;
         n.step_off = io->step_off;
@@ -1572,6 +1575,8 @@ static int launch_node_pass(nfx_ctx* ctx, const nfx_plan& p, int64_t step, const
 struct BatchNodeArgs {
     int64_t N;
     float* x;  // displacements u
+    float* xo;  // where the pass stores u and w (x and w themselves, or the other buffers of a node-fused
+    float* wo;  // call's last step)
     const float* __restrict__ ref;
     float* w;  // velocity-Verlet state w = a v + f/2
     const uint32_t* __restrict__ node_off;
@@ -1598,8 +1603,8 @@ __global__ __launch_bounds__(kBlock) void k_batch_node(BatchNodeArgs a, int64_t 
     node_contacts<SUB, IND>(a.ref, N, n, x, cp->substrate_k, cp->wall, cp->tip_k, cp->tip_radius, pos, f, tf, td);
     V3 w = mk(a.w[n], a.w[N + n], a.w[2 * N + n]);
     vv_update_w(x, w, f);
-    a.x[n] = x.x; a.x[N + n] = x.y; a.x[2 * N + n] = x.z;
-    a.w[n] = w.x; a.w[N + n] = w.y; a.w[2 * N + n] = w.z;
+    a.xo[n] = x.x; a.xo[N + n] = x.y; a.xo[2 * N + n] = x.z;
+    a.wo[n] = w.x; a.wo[N + n] = w.y; a.wo[2 * N + n] = w.z;
 }
 
 // One workgroup per cell: on a sampling step, the cell's indenter force (Simulation.py:198-212 in
@@ -1639,38 +1644,66 @@ static void launch_batch_node_sub(nfx_ctx* ctx, const nfx_plan& p, const BatchNo
     else k_batch_node<SUB, 0><<<nb, kBlock, 0, s>>>(a, step, sd, off);
 }
 
+static int launch_batch_curves(nfx_ctx* ctx, const nfx_plan& p, const nfx_batch& b, const float* x, int64_t step,
+                               const int64_t* sd, int32_t off) {
+    if (p.indenter == NFX_INDENTER_SPHERE)
+        k_batch_curves<1><<<b.ncells, kBlock, 0, ctx->stream>>>(x, p.ref, p.N, b.cell_node_off, b.cells, b.curves,
+                                                                b.ncurve, b.curve_steps, step, sd, off);
+    else
+        k_batch_curves<2><<<b.ncells, kBlock, 0, ctx->stream>>>(x, p.ref, p.N, b.cell_node_off, b.cells, b.curves,
+                                                                b.ncurve, b.curve_steps, step, sd, off);
+    NFX_CHECK_LAUNCH();
+    return NFX_OK;
+}
+
+static int launch_batch_nodes(nfx_ctx* ctx, const nfx_plan& p, const nfx_batch& b, const NodeIO& io, int64_t step,
+                              const int64_t* sd, int32_t off) {
+    const BatchNodeArgs a{p.N, io.x, io.xo, io.vo, p.ref, io.v, p.node_off, io.partials, b.node_cell, b.cells};
+    if (p.substrate) launch_batch_node_sub<true>(ctx, p, a, step, sd, off);
+    else launch_batch_node_sub<false>(ctx, p, a, step, sd, off);
+    NFX_CHECK_LAUNCH();
+    return NFX_OK;
+}
+
+// the batch that a force pass belongs to, set on the context while the pass is enqueued, with the step whose
+// curve samples ride in it (curves)
+struct BatchPass {
+    nfx_ctx* ctx;
+    BatchPass(nfx_ctx* c, const nfx_batch& b, bool curves, int64_t step, const int64_t* sd, int32_t off) : ctx(c) {
+        c->batch = &b;
+        c->curve_fused = curves;
+        c->curve_step = step;
+        c->curve_step_dev = sd;
+        c->curve_off = off;
+    }
+    ~BatchPass() {
+        ctx->batch = nullptr;
+        ctx->curve_fused = false;
+    }
+};
+
 static int launch_batch_step(nfx_ctx* ctx, const nfx_plan& p, const nfx_batch& b, int64_t step, const int64_t* sd,
                              int32_t off, int which = 7) {
     // a whole step enqueues the curve sample inside the force pass's launch (it reads the same
     // positions, before the node pass moves them); the curve pass alone keeps its own kernel
     const bool fuse = (which & 3) == 3 && b.curves;
-    if ((which & 1) && b.curves && !fuse) {
-        if (p.indenter == NFX_INDENTER_SPHERE)
-            k_batch_curves<1><<<b.ncells, kBlock, 0, ctx->stream>>>(p.disp, p.ref, p.N, b.cell_node_off, b.cells,
-                                                                    b.curves, b.ncurve, b.curve_steps, step, sd, off);
-        else
-            k_batch_curves<2><<<b.ncells, kBlock, 0, ctx->stream>>>(p.disp, p.ref, p.N, b.cell_node_off, b.cells,
-                                                                    b.curves, b.ncurve, b.curve_steps, step, sd, off);
-        NFX_CHECK_LAUNCH();
+    int rc = NFX_OK;
+    if ((which & 1) && b.curves && !fuse) rc = launch_batch_curves(ctx, p, b, p.disp, step, sd, off);
+    if (rc == NFX_OK && (which & 2)) {
+        const BatchPass pass(ctx, b, fuse, step, sd, off);
+        rc = launch_force_pass(ctx, p, false);
     }
-    if (which & 2) {
-        ctx->batch = &b;
-        ctx->curve_fused = fuse;
-        ctx->curve_step = step;
-        ctx->curve_step_dev = sd;
-        ctx->curve_off = off;
-        const int rc = launch_force_pass(ctx, p, false);
-        ctx->batch = nullptr;
-        ctx->curve_fused = false;
-        if (rc) return rc;
-    }
-    if (which & 4) {
-        BatchNodeArgs a{p.N, p.disp, p.ref, p.vel, p.node_off, p.partials, b.node_cell, b.cells};
-        if (p.substrate) launch_batch_node_sub<true>(ctx, p, a, step, sd, off);
-        else launch_batch_node_sub<false>(ctx, p, a, step, sd, off);
-        NFX_CHECK_LAUNCH();
-    }
-    return NFX_OK;
+    if (rc == NFX_OK && (which & 4))
+        rc = launch_batch_nodes(ctx, p, b, NodeIO{p.disp, p.disp, p.vel, p.vel, p.partials}, step, sd, off);
+    return rc;
+}
+
+// launch k of a node-fused batch call: the samples of the step it completes ride in it (both read the
+// displacements before that step); a batch keeps w from call to call
+static int launch_batch_fused(nfx_ctx* ctx, const nfx_plan& p, const nfx_batch& b, FusedIO io) {
+    io.vv_first = 0;
+    const BatchPass pass(ctx, b, b.curves != nullptr, io.step, io.step_dev, io.step_off);
+    return launch_fused(ctx, p, false, io);
 }
 
 // ---- captured step blocks --------------------------------------------------------------------
@@ -1716,7 +1749,9 @@ static int capture_graph(nfx_ctx* ctx, const nfx_plan& p, const nfx_batch* b, bo
     }
     int rc = NFX_OK;
     for (int64_t i = 0; i < kGraphBlock && rc == NFX_OK; ++i) {
-        if (b) {
+        if (b && node_fused(p)) {
+            rc = launch_batch_fused(ctx, p, *b, fused_io(p, 2 + i, nullptr, 0, ctx->step_dev, (int32_t)i));
+        } else if (b) {
             rc = launch_batch_step(ctx, p, *b, 0, ctx->step_dev, (int32_t)i);
         } else if (node_fused(p)) {
             // launch i of a block is launch k0 + i of its call with k0 even (run_fused starts blocks at
@@ -1837,6 +1872,39 @@ static int run_fused(nfx_ctx* c, const nfx_plan& p, int64_t step0, int64_t n, do
     const NodeIO io = fused_last_io(p, n);
     return launch_node_pass(c, p, step0 + n - 1, nullptr, 0, tip_hist ? tip_hist + n - 1 : nullptr, nullptr, VV_LAST,
                             &io);
+}
+
+// A node-fused batch call of n >= 2 steps, as run_fused: the same launches, with the curve samples of step
+// k - 1 in launch k and those of the last step ahead of the last node pass
+static int run_fused_batch(nfx_ctx* c, const nfx_plan& p, const nfx_batch& b, int64_t step0, int64_t n, bool use_graph) {
+    int rc = launch_batch_step(c, p, b, step0, nullptr, 0, 2);
+    if (rc) return rc;
+    auto eager = [&](int64_t k) { return launch_batch_fused(c, p, b, fused_io(p, k, nullptr, step0 + k - 1, nullptr, 0)); };
+    rc = eager(1);
+    if (rc) return rc;
+    int64_t k = 2;
+    if (use_graph && n - k >= kGraphBlock) {
+        nfx_ctx::GraphEntry* ge = find_graph(c, p, &b, false);
+        if (!ge) {
+            rc = capture_graph(c, p, &b, false, &ge);
+            if (rc) return rc;
+        }
+        for (; n - k >= kGraphBlock; k += kGraphBlock) {
+            k_set_i64<<<1, 1, 0, c->stream>>>(c->step_dev, step0 + k - 1);
+            NFX_CHECK_LAUNCH();
+            NFX_HIP(hipGraphLaunch(ge->exec, c->stream));
+        }
+    }
+    for (; k < n; ++k) {
+        rc = eager(k);
+        if (rc) return rc;
+    }
+    const NodeIO io = fused_last_io(p, n);
+    if (b.curves) {
+        rc = launch_batch_curves(c, p, b, io.x, step0 + n - 1, nullptr, 0);
+        if (rc) return rc;
+    }
+    return launch_batch_nodes(c, p, b, io, step0 + n - 1, nullptr, 0);
 }
 
 }  // namespace nfx
@@ -2463,6 +2531,7 @@ int nfx_batch_run_steps(nfx_ctx* c, const nfx_plan* p, const nfx_batch* b, int64
     rc = validate_batch(p, b);
     if (rc) return rc;
     NFX_REQUIRE(nsteps >= 0, "nsteps < 0");
+    if (node_fused(*p) && nsteps >= 2) return run_fused_batch(c, *p, *b, step0, nsteps, use_graph != 0);
     int64_t done = 0;
     if (use_graph && nsteps >= kGraphBlock) {  // as in nfx_run_steps: whole blocks replay, the rest is eager
         const int64_t B = kGraphBlock;

@@ -1,0 +1,58 @@
+"""GPU test of the batch's one-launch step (the node update of a step inside the next force pass) against its
+two-launch step: the same operations in the same order, so positions, velocities, plastic state and curves agree bit
+for bit, for calls of one step, two, an odd number, and more than a captured block."""
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+CALLS = (1, 2, 3, 104, 0, 207, 1, 33)
+STEPS = sum(CALLS)
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    import torch
+
+    if not torch.cuda.is_available():
+        pytest.skip("no HIP device")
+    from nofluidx3d_amd import openCL
+
+    openCL.initializeOpenCLObjects(0)
+    return openCL.handle()
+
+
+@pytest.mark.parametrize("viscous,kw", [
+    (False, {}),
+    (False, {"tile_k": 128, "shape_from_ref": False, "narrow": False}),
+    (True, {}),
+    (True, {"tile_k": 512, "use_graph": False}),
+    (True, {"sym_state": False, "plastic_strain": True, "stream_nt": 1}),
+])
+def test_one_launch_steps_match_two_launch_steps(ctx, monkeypatch, viscous, kw):
+    import torch
+
+    from nofluidx3d_amd import autotune
+    from nofluidx3d_amd.batch import BatchSimulation, CellSpec, make_meshes
+
+    specs = [CellSpec(2.5 + 0.5 * i, 0.6, 3100 + i, 300.0 * (i + 1), 0.3 + 0.08 * i, 60.0 if viscous else None, 1.0 + i,
+                      3.0) for i in range(3)]
+    meshes = make_meshes(specs, workers=1, cache=None)
+
+    def run(limit):
+        monkeypatch.setattr(autotune, "NODE_FUSED_MAX_TETRA", limit)
+        b = BatchSimulation(specs, meshes, steps=STEPS, ncurve=50, **kw)
+        assert bool(b.plan.disp_b) == (limit > 0)
+        for _ in range(2):  # again after a reset
+            b.reset(specs)
+            for n in CALLS:
+                b.advance(n)
+            b.sync()
+        out = [b.x, b.v, b.curves] + [t for t in (b.state, b.eps, b.t_active) if t is not None]
+        return [t.clone() for t in out]
+
+    one, two = run(10 ** 9), run(0)
+    assert float(two[2].abs().max()) > 0.0 and bool(torch.isfinite(two[0]).all())
+    for s, t in zip(one, two):
+        assert np.array_equal(s.cpu().numpy(), t.cpu().numpy())
