@@ -47,15 +47,23 @@ def default_stream_nt(tetra):
 # millions of tetra its force pass, which then also updates every node it touches (~2.9 times per
 # node), is longer than the two passes apart.  Measured on MI355X (NH cells, best tile shape of each
 # form, us per graph-replayed step, fused against two launches): 25k tetra 5.5 / 7.2, 106k 6.3 / 7.9,
-# 211k 7.5 / 8.8, 526k 11.7 / 12.5, 878k 16.6 / 16.5; the 3.4M-tetra viscoplastic cell 58 / 50.  Batches,
-# curve samples in the launch (elastic, viscoplastic): 46k 6.2 / 8.2, 6.3 / 8.9; 234k 8.1 / 10.0, 9.2 / 11.5; 780k
-# 15.4 / 15.5, 21.7 / 22.7
+# 211k 7.5 / 8.8, 526k 11.7 / 12.5, 878k 16.6 / 16.5; the 3.4M-tetra viscoplastic cell 58 / 50
 NODE_FUSED_MAX_TETRA = 600_000
+# batches hold out longer: their node pass looks each node's cell up, and the curve samples ride in the one launch.
+# Elastic 46k 6.2 / 8.2, 234k 8.1 / 10.0, 733k 17.8 / 18.1, 887k 20.1 / 19.8, 1.4M 24.2 / 25.0, 2.3M 31.9 / 32.5;
+# viscoplastic 46k 6.3 / 8.9, 234k 9.2 / 11.5, 887k 24.4 / 28.5, 1.4M 33.0 / 34.3, 1.9M 41.8 / 42.2, 2.3M 48.6 / 46.8
+# (cells of 10 k to 100 k tetra, 256-tetra tiles, 43 % of the steps with samples from 733k on)
+BATCH_NODE_FUSED_MAX_TETRA = 2_000_000
 
 
 def default_node_fused(tetra):
-    """the step form of a mesh or batch to use untuned: node-fused for at most NODE_FUSED_MAX_TETRA tetra"""
+    """the step form to use untuned: node-fused for meshes of at most NODE_FUSED_MAX_TETRA tetra"""
     return int(tetra) <= NODE_FUSED_MAX_TETRA
+
+
+def default_batch_node_fused(tetra):
+    """a batch's step form: node-fused for at most BATCH_NODE_FUSED_MAX_TETRA tetra together"""
+    return int(tetra) <= BATCH_NODE_FUSED_MAX_TETRA
 
 
 def group_tetra():

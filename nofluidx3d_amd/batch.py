@@ -31,7 +31,7 @@ import os
 import numpy as np
 
 from nofluidx3d_amd import _lib
-from nofluidx3d_amd.autotune import default_node_fused, default_stream_nt
+from nofluidx3d_amd.autotune import default_batch_node_fused, default_stream_nt
 from nofluidx3d_amd.Simulation import order_tiles, tile_ranges
 
 E_SIM = 1e-2
@@ -344,7 +344,7 @@ class BatchSimulation:
     Q = Fp^-1 - I (9);
     ``narrow`` 16-bit tile-node ids and partial positions (when every cell has < 65536 nodes);
     ``shape_from_ref`` the force pass forms Dm^-1 from the reference positions instead of streaming it.
-    Batches of at most ``autotune.NODE_FUSED_MAX_TETRA`` tetra run the node-fused step (same bits).
+    Batches of at most ``autotune.BATCH_NODE_FUSED_MAX_TETRA`` tetra run the node-fused step (same bits).
 
     State on the device: node displacements u from the FP32 reference positions X0 (``ref``), the
     velocity-Verlet state w = a v + f/2, and for the viscoplastic law the plastic deviation Gd
@@ -371,7 +371,7 @@ class BatchSimulation:
         self.model = _lib.NFX_VISCOPLASTIC if viscous[0] else _lib.NFX_MR
         h = build_host_arrays(specs, meshes, steps, K)
         # one launch per step where launches dominate it, as for single cells (every node a corner of some tetra)
-        fuse = default_node_fused(h["T_real"]) and bool((np.diff(h["node_poff"].astype(np.int64)) > 0).all())
+        fuse = default_batch_node_fused(h["T_real"]) and bool((np.diff(h["node_poff"].astype(np.int64)) > 0).all())
         if not fuse:
             order_batch_tiles(h, K)
         self._meshes = meshes

@@ -41,7 +41,7 @@ def test_one_launch_steps_match_two_launch_steps(ctx, monkeypatch, viscous, kw):
     meshes = make_meshes(specs, workers=1, cache=None)
 
     def run(limit):
-        monkeypatch.setattr(autotune, "NODE_FUSED_MAX_TETRA", limit)
+        monkeypatch.setattr(autotune, "BATCH_NODE_FUSED_MAX_TETRA", limit)
         b = BatchSimulation(specs, meshes, steps=STEPS, ncurve=50, **kw)
         assert bool(b.plan.disp_b) == (limit > 0)
         for _ in range(2):  # again after a reset
