@@ -379,18 +379,17 @@ __device__ __forceinline__ V3 sum_partials8(const float* __restrict__ partials, 
 
 // The contact terms of a node at x = X0 + u, in FP64: the substrate (Substrate.cl:4-5), the
 // indenter (Sphere.cl:9-16 or Plane.cl:4-5) at the FP64 position pos, added to f; the indenter's
-// own force and the penetration for the tip reduction.  X0.x/z and u.x/z are read only for nodes
-// the sphere can touch (y > pos - R): a few per cent of a cell.
-template <bool SUB, int IND>
-__device__ __forceinline__ void node_contacts(const float* __restrict__ ref, int64_t N, int64_t n, V3 u, double sub_k,
-                                              double wall, double ind_k, double ind_radius, double pos, V3& f,
-                                              double& tip_f, double& tip_dis) {
-    const double y = (double)ref[N + n] + (double)u.y;
+// own force and the penetration for the tip reduction.  ry is X0.y, and xz() gives X0.x and X0.z, asked for
+// only at nodes the sphere can touch (y > pos - R): a few per cent of a cell.
+template <bool SUB, int IND, class XZ>
+__device__ __forceinline__ void node_contacts(float ry, XZ&& xz, V3 u, double sub_k, double wall, double ind_k,
+                                              double ind_radius, double pos, V3& f, double& tip_f, double& tip_dis) {
+    const double y = (double)ry + (double)u.y;
     if constexpr (SUB) f.y += (float)(sub_k * fmax(wall - y, 0.0));
     if constexpr (IND == NFX_INDENTER_SPHERE) {
         if (y > pos - ind_radius) {
-            const Contact c = sphere_term_d((double)ref[n] + (double)u.x, y, (double)ref[2 * N + n] + (double)u.z,
-                                            ind_k, ind_radius, pos);
+            const float2 r = xz();
+            const Contact c = sphere_term_d((double)r.x + (double)u.x, y, (double)r.y + (double)u.z, ind_k, ind_radius, pos);
             f = f + mk((float)c.fx, (float)c.fy, (float)c.fz);
             tip_f = -c.fy;
             tip_dis = c.dis;
@@ -429,26 +428,28 @@ struct NodeStep {
 // node n's update (k_node_update's arithmetic, the substrate/indenter/fix choices uniform at run
 // time): x holds u before the step on entry and after it on return; tip receives the node's indenter
 // force when this tile stores the node
-__device__ __forceinline__ void node_step(const NodeStep& s, const ContactConsts& cc, const float* __restrict__ ref,
-                                          int64_t N, uint32_t n, uint32_t dst, uint2 rg, double pos, V3& x,
-                                          double& tip) {
+__device__ __forceinline__ void node_step(const NodeStep& s, const ContactConsts& cc, V3 X0, int64_t N, uint32_t n,
+                                          uint32_t dst, uint2 rg, double pos, V3& x, double& tip) {
     const uint32_t b = rg.x, e = rg.y;
+    // before the partials' sum (and X0 with x): behind the contacts' branches these loads were a memory round of their
+    // own (steps of a 105 k tetra cell 6.7 -> 6.4 us, of a 0.5 M one 17.5 -> 16.9, of 32 cells of together 1.4 M 32 -> 30)
+    V3 w = mk(s.w[n], s.w[N + n], s.w[2 * N + n]);
     V3 f = sum_partials8(s.prev_partials, b, e);
+    auto xz = [&] { return make_float2(X0.x, X0.z); };
     double tf = 0.0, td = 0.0;
     if (s.substrate) {
         if (s.indenter == NFX_INDENTER_SPHERE)
-            node_contacts<true, NFX_INDENTER_SPHERE>(ref, N, n, x, cc.sub_k, cc.wall, cc.ind_k, cc.ind_radius, pos, f, tf, td);
+            node_contacts<true, NFX_INDENTER_SPHERE>(X0.y, xz, x, cc.sub_k, cc.wall, cc.ind_k, cc.ind_radius, pos, f, tf, td);
         else if (s.indenter == NFX_INDENTER_PLANE)
-            node_contacts<true, NFX_INDENTER_PLANE>(ref, N, n, x, cc.sub_k, cc.wall, cc.ind_k, cc.ind_radius, pos, f, tf, td);
+            node_contacts<true, NFX_INDENTER_PLANE>(X0.y, xz, x, cc.sub_k, cc.wall, cc.ind_k, cc.ind_radius, pos, f, tf, td);
         else
-            node_contacts<true, NFX_INDENTER_NONE>(ref, N, n, x, cc.sub_k, cc.wall, cc.ind_k, cc.ind_radius, pos, f, tf, td);
+            node_contacts<true, NFX_INDENTER_NONE>(X0.y, xz, x, cc.sub_k, cc.wall, cc.ind_k, cc.ind_radius, pos, f, tf, td);
     } else {
         if (s.indenter == NFX_INDENTER_SPHERE)
-            node_contacts<false, NFX_INDENTER_SPHERE>(ref, N, n, x, cc.sub_k, cc.wall, cc.ind_k, cc.ind_radius, pos, f, tf, td);
+            node_contacts<false, NFX_INDENTER_SPHERE>(X0.y, xz, x, cc.sub_k, cc.wall, cc.ind_k, cc.ind_radius, pos, f, tf, td);
         else if (s.indenter == NFX_INDENTER_PLANE)
-            node_contacts<false, NFX_INDENTER_PLANE>(ref, N, n, x, cc.sub_k, cc.wall, cc.ind_k, cc.ind_radius, pos, f, tf, td);
+            node_contacts<false, NFX_INDENTER_PLANE>(X0.y, xz, x, cc.sub_k, cc.wall, cc.ind_k, cc.ind_radius, pos, f, tf, td);
     }
-    V3 w = mk(s.w[n], s.w[N + n], s.w[2 * N + n]);
     if (s.vv_first) {
         w = vv_w_from_v(w, f, mk(s.fold[n], s.fold[N + n], s.fold[2 * N + n]));
         x = x + w;
@@ -456,8 +457,8 @@ __device__ __forceinline__ void node_step(const NodeStep& s, const ContactConsts
         vv_update_w(x, w, f);
     }
     if (s.fix && (n == 3 || n == 4)) {  // x = z = 0 (VelocityVerlet.cl:17-22): u = -X0
-        x.x = -ref[n];
-        x.z = -ref[2 * N + n];
+        x.x = -X0.x;
+        x.z = -X0.z;
     }
     if (dst == b) {
         s.x_next[n] = x.x; s.x_next[N + n] = x.y; s.x_next[2 * N + n] = x.z;
@@ -477,8 +478,8 @@ __device__ __forceinline__ void node_step(const NodeStep& s, const ContactConsts
 // runs of one length then read different LDS banks at every step (2.65 M tetra cell: bank conflicts 6.5 M -> 4.3 M
 // of 12.1 M -> 9.6 M LDS cycles per launch, step -2 to -3 %).  A node-fused launch also gathers and stores its
 // nodes and lost 1.6 % to the order: its lists keep ascending ids.  Phases:
-//   0  issue the tetra's streaming loads (Dm^-1 and V0 unless GEO, the viscoplastic state and epsbar),
-//      its corner records and the tile metadata
+//   0  issue the loads of the tetra's corner records and of the tile metadata, then its streaming loads (Dm^-1 and
+//      V0 unless GEO, the viscoplastic state and epsbar)
 //   1  node displacements (GEO: and reference positions) and run starts -> LDS
 //   2  (GEO: Dm^-1 and V0 from the reference edges) material law on LDS displacements; each corner
 //      force -> LDS at its place in the sorted list
@@ -511,7 +512,7 @@ struct TileArgs {
     const uint16_t* __restrict__ tile_ntet;
     const uint32_t* __restrict__ tile_cell;
     const nfx_cell* __restrict__ cells;
-    // batches (NARROW): tile-node ids and partial positions as 16-bit offsets from per-tile bases
+    // batches (META 2): tile-node ids and partial positions as 16-bit offsets from per-tile bases
     const uint16_t* __restrict__ tile_nodes16;
     const uint16_t* __restrict__ tile_dst16;
     const uint32_t* __restrict__ tile_node_base;
@@ -589,15 +590,19 @@ __host__ __device__ constexpr size_t tile_lds_bytes(int K, int max_nodes, bool g
     return (size_t)12 * tile_corner_slots(K, node) + (size_t)(16 + (geo ? 8 : 0) + 2) * max_nodes;
 }
 
+// A cell's kernels know nothing of batches: the tests for curve samples and cell constants, uniform as they are, put a
+// fetch of kernel arguments ahead of the first loads (step of a 0.5 M tetra cell with flow 16.2 -> 15.8 us)
+enum { META_CELL = 0, META_BATCH = 1, META_BATCH16 = 2 };
+
 // GEO: Dm^-1 and V0 from the staged reference positions; NT: cache policy of the streams; EPS: the
 // viscoplastic law keeps its accumulated plastic strain (the linear law does not read it); SYM: its
-// state is the symmetric deviation Gd (6 planes) instead of Q (9 planes); NARROW: 16-bit tile-node
-// metadata (batches); NODE: the previous step's node update rides in this pass.  Waves per SIMD: the
+// state is the symmetric deviation Gd (6 planes) instead of Q (9 planes); META: 0 a single
+// cell, 1 a batch, 2 a batch with 16-bit tile-node metadata; NODE: the previous step's node update rides in this pass.  Waves per SIMD: the
 // viscoplastic forms fit 72 VGPRs (7 waves; measured 5 % faster than 6, while the 64-register bound
 // of 8 waves spills and is slower) except with stress outputs or NODE (6), and the symmetric one
 // without epsbar fits 64 (8 waves)
 template <int MODEL, int K, bool GEO, bool STRESS, bool NT = false, bool EPS = true, bool SYM = false,
-          bool NARROW = false, bool NODE = false>
+          int META = META_CELL, bool NODE = false>
 __global__ __launch_bounds__(K, MODEL != NFX_VISCOPLASTIC ? 8 : (STRESS || NODE) ? 6 : (!SYM || EPS) ? 7 : 8) void k_tile_force(TileArgs a, ElasticDev e, VPConst P, float* __restrict__ Sst,
                                                   float* __restrict__ eps, float* __restrict__ vm,
                                                   float* __restrict__ pr) {
@@ -617,8 +622,8 @@ __global__ __launch_bounds__(K, MODEL != NFX_VISCOPLASTIC ? 8 : (STRESS || NODE)
     // the step's curve samples go first: a sample is one workgroup's chain of memory rounds, which the tiles
     // then hide.  At the end of the grid it was the launch's tail: steps of 32 cells of together 1.4 M tetra, 43 % of
     // them with samples, 41.7 -> 33.0 us.  Padded to a multiple of 8, so that the node pass's XCD ranges stay the tiles'
-    const uint32_t first_tile = ((uint32_t)a.curve_blocks + 7u) & ~7u;
-    if (blockIdx.x < first_tile) {
+    const uint32_t first_tile = META ? ((uint32_t)a.curve_blocks + 7u) & ~7u : 0u;
+    if (META && blockIdx.x < first_tile) {
         if (blockIdx.x >= (uint32_t)a.curve_blocks) return;
         const int64_t time = a.curve_step_dev ? (*a.curve_step_dev + a.curve_off) : a.curve_step;
         batch_curve_sample(a.x, a.ref, a.N, a.cell_node_off, a.cells, a.curves, a.ncurve, a.curve_steps, time,
@@ -628,9 +633,36 @@ __global__ __launch_bounds__(K, MODEL != NFX_VISCOPLASTIC ? 8 : (STRESS || NODE)
     const int64_t c = xcd_block(blockIdx.x - first_tile, gridDim.x - first_tile);
     const int64_t T = a.T, N = a.N;
     const int64_t t0 = c * K;
+    const int tl = threadIdx.x;
+    const uint32_t u = (uint32_t)tl;
+    // what the chain of loads hangs on goes first, the state's streams behind it and not ahead (step of a 0.5 M tetra
+    // cell with flow 16.9 -> 16.2 us, of 32 cells of together 1.4 M 29.7 -> 28.8).  This tetra's 4 corner records (tile-node | rank << 8), as one
+    // 8-byte load (whole tiles are stored), and the tile metadata: thread tl owns tile-node tl (MX <= K, checked on
+    // the host)
+    const uint64_t cr = ld_g<NT, uint64_t>(uat(reinterpret_cast<const uint64_t*>(a.tile_corners + 4 * K * c), u));
+    const int64_t j0 = c * (int64_t)MX;
+    const bool owner = tl < MX;
+    uint32_t nid = 0, dst = 0;
+    int lb = 0, le = 0;
+    uint2 rg = make_uint2(0u, 0u);  // NODE: the node's partials of the previous force pass
+    if (owner) {
+        if constexpr (NODE) rg = a.ns.range[j0 + tl];
+        if constexpr (META == META_BATCH16) {
+            nid = a.tile_node_base[c] + (uint32_t)ld_g<NT, uint16_t>(uat(a.tile_nodes16 + j0, u));
+            dst = a.tile_dst_base[c] + (uint32_t)ld_g<NT, uint16_t>(uat(a.tile_dst16 + j0, u));
+        } else {
+            nid = ld_g<NT, uint32_t>(uat(a.tile_nodes + j0, u));
+            dst = ld_g<NT, uint32_t>(uat(a.tile_dst + j0, u));
+        }
+        lb = tl ? ld_g<NT, uint16_t>(uat(a.tile_lend + j0, u - 1)) : 0;
+        if constexpr (!NODE) lb += (lb ^ tl) & a.odd;  // the first place of the run's parity
+        le = ld_g<NT, uint16_t>(uat(a.tile_lend + j0, u));
+    }
+    // scalar loads, in flight with them: the tile's node count, its cell, its flag and the step
+    const int M = (int)a.tile_count[c];
     int nt = (int)((T - t0) < K ? (T - t0) : K);
     ContactConsts cc = a.ns.cc;  // NODE
-    if (a.cells) {  // batch: this tile's cell and its constants (uniform over the workgroup)
+    if constexpr (META != META_CELL) {  // this tile's cell and its constants (uniform over the workgroup)
         nt = a.tile_ntet[c];
         const nfx_cell cp = a.cells[a.tile_cell[c]];
         if constexpr (NODE)
@@ -646,16 +678,19 @@ __global__ __launch_bounds__(K, MODEL != NFX_VISCOPLASTIC ? 8 : (STRESS || NODE)
         P.sy = cp.vp_offset;
         P.linear = 1;
     }
-    const int tl = threadIdx.x;
+    double pos = 0.0;  // NODE: the indenter's position in the step being completed
+    if constexpr (NODE) {
+        const int64_t time = a.ns.step_dev ? (*a.ns.step_dev + a.ns.step_off) : a.ns.step;
+        pos = indenter_pos(cc.ind_start, cc.ind_speed, cc.ind_move, time);
+    }
     const bool active = tl < nt;
-    const uint32_t u = (uint32_t)tl;
     // the tile's plastic-activity flag (uniform): without it every tile reads its state
     bool plastic = true;
     if constexpr (MODEL == NFX_VISCOPLASTIC) {
         if (a.vp_active) plastic = a.vp_active[c] != 0u;
     }
 
-    // issue this tetra's streaming loads first: they overlap the staging phases below
+    // this tetra's streaming loads: they overlap the staging phases below
     float D[9], Sv[MODEL == NFX_VISCOPLASTIC ? 9 : 1], e0 = 0.f, v0 = 0.f, sdm = 0.f;
     if (active) {
         if constexpr (!GEO) {
@@ -676,49 +711,22 @@ __global__ __launch_bounds__(K, MODEL != NFX_VISCOPLASTIC ? 8 : (STRESS || NODE)
             v0 = ld_g<NT, float>(uat(a.v0 + t0, u));
         }
     }
-
-    // tile metadata: thread tl owns tile-node tl (MX <= K, checked on the host)
-    const int64_t j0 = c * (int64_t)MX;
-    const int M = (int)a.tile_count[c];
-    const bool owner = tl < MX;
-    uint32_t nid = 0, dst = 0;
-    int lb = 0, le = 0;
-    uint2 rg = make_uint2(0u, 0u);  // NODE: the node's partials of the previous force pass
-    if (owner) {
-        if constexpr (NODE) rg = a.ns.range[j0 + tl];
-        if constexpr (NARROW) {
-            nid = a.tile_node_base[c] + (uint32_t)ld_g<NT, uint16_t>(uat(a.tile_nodes16 + j0, u));
-            dst = a.tile_dst_base[c] + (uint32_t)ld_g<NT, uint16_t>(uat(a.tile_dst16 + j0, u));
-        } else {
-            nid = ld_g<NT, uint32_t>(uat(a.tile_nodes + j0, u));
-            dst = ld_g<NT, uint32_t>(uat(a.tile_dst + j0, u));
-        }
-        lb = tl ? ld_g<NT, uint16_t>(uat(a.tile_lend + j0, u - 1)) : 0;
-        if constexpr (!NODE) lb += (lb ^ tl) & a.odd;  // the first place of the run's parity
-        le = ld_g<NT, uint16_t>(uat(a.tile_lend + j0, u));
-    }
-    // this tetra's 4 corner records (tile-node | rank << 8), as one 8-byte load
-    uint64_t cr = 0;
-    if (active) cr = ld_g<NT, uint64_t>(uat(reinterpret_cast<const uint64_t*>(a.tile_corners + 4 * K * c), u));
     double tip = 0.0;  // NODE: the indenter force on the node this thread stores
     if (owner) {
         float ux = a.x[nid], uy = a.x[N + nid], uz = a.x[2 * N + nid];
+        V3 X0 = mk(0.f, 0.f, 0.f);
+        if constexpr (GEO || NODE) X0 = mk(a.ref[nid], a.ref[N + nid], a.ref[2 * N + nid]);
         if (NODE && tl < M) {  // complete the previous step at this node (padding entries past M are
                                // not nodes of the tile); the forces below see the result
-            double pos = 0.0;
-            if (a.ns.indenter) {
-                const int64_t time = a.ns.step_dev ? (*a.ns.step_dev + a.ns.step_off) : a.ns.step;
-                pos = indenter_pos(cc.ind_start, cc.ind_speed, cc.ind_move, time);
-            }
             V3 xn = mk(ux, uy, uz);
-            node_step(a.ns, cc, a.ref, N, nid, dst, rg, pos, xn, tip);
+            node_step(a.ns, cc, X0, N, nid, dst, rg, pos, xn, tip);
             ux = xn.x;
             uy = xn.y;
             uz = xn.z;
         }
         if constexpr (GEO) {
-            s_n[tl] = make_float4(ux, uy, uz, a.ref[nid]);
-            s_r[tl] = make_float2(a.ref[N + nid], a.ref[2 * N + nid]);
+            s_n[tl] = make_float4(ux, uy, uz, X0.x);
+            s_r[tl] = make_float2(X0.y, X0.z);
         } else {
             s_n[tl] = make_float4(ux, uy, uz, 0.0f);
         }
@@ -974,6 +982,11 @@ __global__ __launch_bounds__(kBlock) void k_node_update(NodeArgs a, int64_t step
     // XCD-aware block order, as the tile force pass has it: an XCD updates the contiguous node range
     // whose partials its own tiles wrote (nodes and tetra follow one Morton order); -2.5 % per launch
     for (int64_t n = (xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x) / G; n < N; n += stride) {
+        // the node's own state first: these loads are then in flight with the gather's instead of behind it
+        // (40 steps of a 215 k tetra cell on corner records 537 -> 523 us)
+        V3 x = mk(a.x[n], a.x[N + n], a.x[2 * N + n]);
+        V3 v = mk(a.v[n], a.v[N + n], a.v[2 * N + n]);  // v, or w inside a call
+        const float ry = SUB || IND ? a.ref[N + n] : 0.0f;
         V3 f;
         if constexpr (GATHER == 1) {
             f = gather_node<G>(a, n, sub);
@@ -983,14 +996,13 @@ __global__ __launch_bounds__(kBlock) void k_node_update(NodeArgs a, int64_t step
             f = mk(a.force[n], a.force[N + n], a.force[2 * N + n]);
         }
         if (sub != 0) continue;
-        V3 x = mk(a.x[n], a.x[N + n], a.x[2 * N + n]);
         double tf = 0.0, td = 0.0;
-        node_contacts<SUB, IND>(a.ref, N, n, x, a.sub_k, a.wall, a.ind_k, a.ind_radius, pos, f, tf, td);
+        node_contacts<SUB, IND>(ry, [&] { return make_float2(a.ref[n], a.ref[2 * N + n]); }, x, a.sub_k, a.wall, a.ind_k,
+                                a.ind_radius, pos, f, tf, td);
         if constexpr (TIP) {
             tsum += tf;
             tmax = fmax(tmax, td);
         }
-        V3 v = mk(a.v[n], a.v[N + n], a.v[2 * N + n]);  // v, or w inside a call
         if constexpr (VVM == VV_PLAIN) {
             vv_update(x, v, f, mk(a.fold[n], a.fold[N + n], a.fold[2 * N + n]));
         } else if constexpr (VVM == VV_FIRST) {
@@ -1235,36 +1247,30 @@ static void launch_tile_legacy(unsigned int nb, size_t lds, hipStream_t s, const
         k_tile_force<MODEL, K, GEO, false><<<nb, K, lds, s>>>(a, e, c, nullptr, nullptr, nullptr, nullptr);
 }
 
-template <int K, bool GEO, bool STRESS, bool NT, bool NODE>
-static void launch_tile_vp(unsigned int nb, size_t lds, hipStream_t s, const TileArgs& a, const ElasticDev& e,
+// the laws with both cache policies
+template <int MODEL, int K, bool GEO, bool STRESS, bool EPS, bool SYM, int META, bool NODE>
+static void launch_tile_nt(unsigned int nb, size_t lds, hipStream_t s, const TileArgs& a, const ElasticDev& e,
                            const VPConst& c, const nfx_plan& p) {
     float* vm = STRESS ? p.von_mises : nullptr;
     float* pr = STRESS ? p.pressure : nullptr;
-    if constexpr (!STRESS && !NODE) {  // the batch's form: symmetric state with 16-bit tile-node metadata
-        if (p.vp_sym && a.tile_nodes16) {
-            if (p.epsbar)
-                k_tile_force<NFX_VISCOPLASTIC, K, GEO, false, NT, true, true, true><<<nb, K, lds, s>>>(a, e, c, p.vp_state,
-                                                                                                p.epsbar, vm, pr);
-            else
-                k_tile_force<NFX_VISCOPLASTIC, K, GEO, false, NT, false, true, true><<<nb, K, lds, s>>>(a, e, c, p.vp_state,
-                                                                                                 nullptr, vm, pr);
-            return;
-        }
-    }
+    float* st = MODEL == NFX_VISCOPLASTIC ? p.vp_state : nullptr;
+    float* eps = MODEL == NFX_VISCOPLASTIC && EPS ? p.epsbar : nullptr;
+    if (p.stream_nt)
+        k_tile_force<MODEL, K, GEO, STRESS, true, EPS, SYM, META, NODE><<<nb, K, lds, s>>>(a, e, c, st, eps, vm, pr);
+    else
+        k_tile_force<MODEL, K, GEO, STRESS, false, EPS, SYM, META, NODE><<<nb, K, lds, s>>>(a, e, c, st, eps, vm, pr);
+}
+
+template <int K, bool GEO, bool STRESS, int META, bool NODE>
+static void launch_tile_vp(unsigned int nb, size_t lds, hipStream_t s, const TileArgs& a, const ElasticDev& e,
+                           const VPConst& c, const nfx_plan& p) {
     constexpr int VP = NFX_VISCOPLASTIC;
     if (p.vp_sym) {
-        if (p.epsbar)
-            k_tile_force<VP, K, GEO, STRESS, NT, true, true, false, NODE><<<nb, K, lds, s>>>(a, e, c, p.vp_state,
-                                                                                       p.epsbar, vm, pr);
-        else
-            k_tile_force<VP, K, GEO, STRESS, NT, false, true, false, NODE><<<nb, K, lds, s>>>(a, e, c, p.vp_state,
-                                                                                        nullptr, vm, pr);
-    } else if (p.epsbar) {
-        k_tile_force<VP, K, GEO, STRESS, NT, true, false, false, NODE><<<nb, K, lds, s>>>(a, e, c, p.vp_state, p.epsbar,
-                                                                                    vm, pr);
-    } else {
-        k_tile_force<VP, K, GEO, STRESS, NT, false, false, false, NODE><<<nb, K, lds, s>>>(a, e, c, p.vp_state, nullptr,
-                                                                                     vm, pr);
+        if (p.epsbar) launch_tile_nt<VP, K, GEO, STRESS, true, true, META, NODE>(nb, lds, s, a, e, c, p);
+        else launch_tile_nt<VP, K, GEO, STRESS, false, true, META, NODE>(nb, lds, s, a, e, c, p);
+    } else if constexpr (META != META_BATCH16) {
+        if (p.epsbar) launch_tile_nt<VP, K, GEO, STRESS, true, false, META, NODE>(nb, lds, s, a, e, c, p);
+        else launch_tile_nt<VP, K, GEO, STRESS, false, false, META, NODE>(nb, lds, s, a, e, c, p);
     }
 }
 
@@ -1340,46 +1346,40 @@ static void launch_tiled_k(nfx_ctx* ctx, const nfx_plan& p, bool st, const Fused
     hipStream_t s = ctx->stream;
     float* vm = st ? p.von_mises : nullptr;
     float* pr = st ? p.pressure : nullptr;
-    const bool nt = p.stream_nt != 0;
+    constexpr int MR = NFX_MR;
+    if (ctx->batch) {  // MR or viscoplastic, no stress outputs (validate_batch)
+        // 16-bit metadata for the two-launch step's elastic law and symmetric state
+        if constexpr (!NODE) {
+            if (a.tile_nodes16 && (p.model == MR || p.vp_sym)) {
+                if (p.model == MR) launch_tile_nt<MR, K, GEO, false, true, false, META_BATCH16, false>(nb, lds, s, a, e, c, p);
+                else launch_tile_vp<K, GEO, false, META_BATCH16, false>(nb, lds, s, a, e, c, p);
+                return;
+            }
+        }
+        if (p.model == MR) launch_tile_nt<MR, K, GEO, false, true, false, META_BATCH, NODE>(nb, lds, s, a, e, c, p);
+        else launch_tile_vp<K, GEO, false, META_BATCH, NODE>(nb, lds, s, a, e, c, p);
+        return;
+    }
     if constexpr (NODE) {  // the single-cell laws of a node-fused step (validate_plan admits no other)
         constexpr bool N_ = true;
         switch (p.model) {
-            case NFX_MR:
-                if (nt)
-                    k_tile_force<NFX_MR, K, GEO, false, true, true, false, false, N_><<<nb, K, lds, s>>>(a, e, c, nullptr,
-                                                                                             nullptr, nullptr, nullptr);
-                else
-                    k_tile_force<NFX_MR, K, GEO, false, false, true, false, false, N_><<<nb, K, lds, s>>>(a, e, c, nullptr,
-                                                                                              nullptr, nullptr, nullptr);
-                break;
+            case NFX_MR: launch_tile_nt<MR, K, GEO, false, true, false, META_CELL, true>(nb, lds, s, a, e, c, p); break;
             case NFX_SVK:
-                k_tile_force<NFX_SVK, K, GEO, false, false, true, false, false, N_><<<nb, K, lds, s>>>(a, e, c, nullptr,
-                                                                                           nullptr, nullptr, nullptr);
+                k_tile_force<NFX_SVK, K, GEO, false, false, true, false, META_CELL, N_><<<nb, K, lds, s>>>(
+                    a, e, c, nullptr, nullptr, nullptr, nullptr);
                 break;
             case NFX_SVKK:
-                k_tile_force<NFX_SVKK, K, GEO, false, false, true, false, false, N_><<<nb, K, lds, s>>>(a, e, c, nullptr,
-                                                                                            nullptr, nullptr, nullptr);
+                k_tile_force<NFX_SVKK, K, GEO, false, false, true, false, META_CELL, N_><<<nb, K, lds, s>>>(
+                    a, e, c, nullptr, nullptr, nullptr, nullptr);
                 break;
             default:
-                if (st && nt) launch_tile_vp<K, GEO, true, true, true>(nb, lds, s, a, e, c, p);
-                else if (st) launch_tile_vp<K, GEO, true, false, true>(nb, lds, s, a, e, c, p);
-                else if (nt) launch_tile_vp<K, GEO, false, true, true>(nb, lds, s, a, e, c, p);
-                else launch_tile_vp<K, GEO, false, false, true>(nb, lds, s, a, e, c, p);
+                if (st) launch_tile_vp<K, GEO, true, META_CELL, true>(nb, lds, s, a, e, c, p);
+                else launch_tile_vp<K, GEO, false, META_CELL, true>(nb, lds, s, a, e, c, p);
         }
         return;
     }
     switch (p.model) {
-        case NFX_MR:
-            if (a.tile_nodes16 && nt)
-                k_tile_force<NFX_MR, K, GEO, false, true, true, false, true><<<nb, K, lds, s>>>(a, e, c, nullptr, nullptr,
-                                                                                         nullptr, nullptr);
-            else if (a.tile_nodes16)
-                k_tile_force<NFX_MR, K, GEO, false, false, true, false, true><<<nb, K, lds, s>>>(a, e, c, nullptr, nullptr,
-                                                                                          nullptr, nullptr);
-            else if (nt)
-                k_tile_force<NFX_MR, K, GEO, false, true><<<nb, K, lds, s>>>(a, e, c, nullptr, nullptr, nullptr, nullptr);
-            else k_tile_force<NFX_MR, K, GEO, false><<<nb, K, lds, s>>>(a, e, c, nullptr, nullptr, nullptr, nullptr);
-            break;
+        case NFX_MR: launch_tile_nt<MR, K, GEO, false, true, false, META_CELL, false>(nb, lds, s, a, e, c, p); break;
         case NFX_SVK: k_tile_force<NFX_SVK, K, GEO, false><<<nb, K, lds, s>>>(a, e, c, nullptr, nullptr, nullptr, nullptr); break;
         case NFX_SVKK: k_tile_force<NFX_SVKK, K, GEO, false><<<nb, K, lds, s>>>(a, e, c, nullptr, nullptr, nullptr, nullptr); break;
         case NFX_LINEAR_ELASTIC: launch_tile_legacy<NFX_LINEAR_ELASTIC, K, GEO>(nb, lds, s, a, e, c, vm, pr); break;
@@ -1387,10 +1387,8 @@ static void launch_tiled_k(nfx_ctx* ctx, const nfx_plan& p, bool st, const Fused
         case NFX_NEO_HOOKEAN_2: launch_tile_legacy<NFX_NEO_HOOKEAN_2, K, GEO>(nb, lds, s, a, e, c, vm, pr); break;
         case NFX_PORO_NEO_HOOKEAN: launch_tile_legacy<NFX_PORO_NEO_HOOKEAN, K, GEO>(nb, lds, s, a, e, c, vm, pr); break;
         default:
-            if (st && nt) launch_tile_vp<K, GEO, true, true, false>(nb, lds, s, a, e, c, p);
-            else if (st) launch_tile_vp<K, GEO, true, false, false>(nb, lds, s, a, e, c, p);
-            else if (nt) launch_tile_vp<K, GEO, false, true, false>(nb, lds, s, a, e, c, p);
-            else launch_tile_vp<K, GEO, false, false, false>(nb, lds, s, a, e, c, p);
+            if (st) launch_tile_vp<K, GEO, true, META_CELL, false>(nb, lds, s, a, e, c, p);
+            else launch_tile_vp<K, GEO, false, META_CELL, false>(nb, lds, s, a, e, c, p);
     }
 }
 
@@ -1595,13 +1593,15 @@ __global__ __launch_bounds__(kBlock) void k_batch_node(BatchNodeArgs a, int64_t 
     const int64_t N = a.N;
     const int64_t n = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;  // XCD-aware, as k_node_update
     if (n >= N) return;
-    V3 f = sum_partials8(a.partials, a.node_off[n], a.node_off[n + 1]);
+    V3 x = mk(a.x[n], a.x[N + n], a.x[2 * N + n]);  // its own state first, as k_node_update
+    V3 w = mk(a.w[n], a.w[N + n], a.w[2 * N + n]);
+    const float ry = a.ref[N + n];
     const nfx_cell* cp = a.cells + a.node_cell[n];
-    V3 x = mk(a.x[n], a.x[N + n], a.x[2 * N + n]);
+    V3 f = sum_partials8(a.partials, a.node_off[n], a.node_off[n + 1]);
     const double pos = IND ? indenter_pos(cp->tip_start, cp->tip_speed, cp->tip_move_steps, time) : 0.0;
     double tf = 0.0, td = 0.0;
-    node_contacts<SUB, IND>(a.ref, N, n, x, cp->substrate_k, cp->wall, cp->tip_k, cp->tip_radius, pos, f, tf, td);
-    V3 w = mk(a.w[n], a.w[N + n], a.w[2 * N + n]);
+    node_contacts<SUB, IND>(ry, [&] { return make_float2(a.ref[n], a.ref[2 * N + n]); }, x, cp->substrate_k, cp->wall,
+                            cp->tip_k, cp->tip_radius, pos, f, tf, td);
     vv_update_w(x, w, f);
     a.xo[n] = x.x; a.xo[N + n] = x.y; a.xo[2 * N + n] = x.z;
     a.wo[n] = w.x; a.wo[N + n] = w.y; a.wo[2 * N + n] = w.z;
