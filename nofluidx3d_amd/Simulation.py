@@ -34,7 +34,7 @@ import time
 import numpy as np
 
 from nofluidx3d_amd import _lib, openCL
-from nofluidx3d_amd.autotune import default_stream_nt
+from nofluidx3d_amd.autotune import default_node_fused, default_stream_nt
 from nofluidx3d_amd.interactions import (FiniteStrainViscoplastic, LegacyElastic, LinearElastic,
                                         LinearElasticDeviatoric, LinearViscoelastic, Plane, PoroNeoHookean,
                                         SecondOrderNeoHookean, Sphere, Substrate, Tetra, VelocityVerlet)
@@ -658,8 +658,6 @@ class Simulation:
         """whether the fused tiled step should take the node-fused form (fuse_node_pass, or by mesh
         size when it is None)"""
         if self.fuse_node_pass is None:
-            from nofluidx3d_amd.autotune import default_node_fused
-
             return default_node_fused(self.numTetra)
         return bool(self.fuse_node_pass)
 

@@ -223,6 +223,7 @@ SIGNATURES = {
 }
 
 _lib = None
+_entries = {}
 _extra_signatures = []
 
 
@@ -260,10 +261,16 @@ def check(rc: int, what: str = ""):
 def call(name: str, *args):
     """Call ``name`` and raise NfxError on a non-zero return.  The argument count is checked
     against the declared signature (ctypes would pass surplus arguments on silently)."""
-    want = len(SIGNATURES[name][1])
+    entry = _entries.get(name)
+    if entry is None:
+        # an entry point and its argument count, looked up once: a per-plugin step makes five calls of ~2 us each
+        entry = _entries[name] = (getattr(lib(), name), len(SIGNATURES[name][1]))
+    fn, want = entry
     if len(args) != want:
         raise TypeError(f"{name} takes {want} arguments ({len(args)} given)")
-    check(getattr(lib(), name)(*args), name)
+    rc = fn(*args)
+    if rc:
+        check(rc, name)
 
 
 def ptr(t) -> int:

@@ -19,6 +19,8 @@ Two hooks belong to this implementation:
 
 from __future__ import annotations
 
+from nofluidx3d_amd import _lib, openCL
+
 
 class DeviceCall:
     """A libnfx entry point bound to an argument provider: ``call()`` enqueues it on the active
@@ -30,8 +32,6 @@ class DeviceCall:
         self.args = args
 
     def __call__(self):
-        from nofluidx3d_amd import _lib, openCL
-
         _lib.call(self.entry, openCL.handle(), *self.args())
 
 

@@ -22,7 +22,7 @@ import math
 
 import numpy as np
 
-from nofluidx3d_amd import _lib
+from nofluidx3d_amd import _lib, openCL
 
 LR, BETA1, BETA2, EPS = 1e-3, 0.9, 0.999, 1e-8
 
@@ -106,8 +106,6 @@ class MLP:
     @staticmethod
     def _gemm(epi, M, N, K, A, lda, B, ldb, bias=None, C=None, Z=None, H=None, HT=None, m=None, v=None, lr_t=0.0,
               bc2=1.0, grad_scale=1.0, split=1, ws=None):
-        from nofluidx3d_amd import openCL
-
         p = lambda t: None if t is None else t.data_ptr()
         g = _lib.MlpGemm(epi, M, N, K, p(A), lda, p(B), ldb, p(bias), p(C), p(Z), p(H), p(HT), p(m), p(v),
                          lr_t, bc2, BETA1, BETA2, EPS, grad_scale, p(ws) if split > 1 else None, split)
@@ -157,8 +155,6 @@ class MLP:
 
     def sync(self):
         import torch
-
-        from nofluidx3d_amd import openCL
 
         _lib.call("nfx_stream_sync", openCL.handle())
         torch.cuda.synchronize(self.dev)
