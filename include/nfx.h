@@ -363,8 +363,9 @@ int nfx_hard_adhesive_plane_surface_force(nfx_ctx* ctx, float* force, const floa
  *      indenter terms at the device-computed indenter position (Simulation.py:117-132, 173-183)
  *      and the damped velocity-Verlet update, on the displacement state (plan.ref, plan.disp).
  *      tip_hist (device, nullable, nsteps doubles) receives the FP64 indenter force of each step.
- *      use_graph != 0 replays whole blocks of 100 steps from a captured hipGraph (captured once per
- *      plan and history mode, and reused whatever nsteps is); the remainder runs eagerly.
+ *      use_graph != 0 replays whole blocks of 96 steps from a captured hipGraph (captured once per
+ *      plan and history mode, by the first call of two blocks or the second of one, and reused whatever nsteps is);
+ *      the remainder runs eagerly, and so does a call on a stream that its caller is capturing.
  *      Between calls the velocity-Verlet state is the reference's (vel, fold).  Inside a call of
  *      n >= 2 steps the first step turns it into w = a v + f_old/2 (kept in vel), the middle steps
  *      advance (disp, w) without a previous force (24 B per node less), and the last step turns w
@@ -373,7 +374,7 @@ int nfx_hard_adhesive_plane_surface_force(nfx_ctx* ctx, float* force, const floa
  *      (disp_b, vel_b, partials_b), steps 1 .. n-1 of the call are one launch each (the node update
  *      of the step before rides in the force pass) and a last node pass ends the call; the first
  *      call with a tip history allocates the context's per-tile indenter-force rows (ceil(T/tile_k)
- *      x 100 doubles), so a caller that captures this call makes one such call beforehand. ------ */
+ *      x 96 doubles), so a caller that captures this call makes one such call beforehand. ------ */
 int nfx_run_steps(nfx_ctx* ctx, const nfx_plan* plan, int64_t step0, int64_t nsteps, double* tip_hist,
                   int32_t use_graph);
 /* number of step blocks the context has captured into graphs so far (a replay of a cached block

@@ -8,7 +8,7 @@ Stepping.  When the registered plugins form the reference's standard chain -- on
 (Tetra or FiniteStrainViscoplastic), optionally a Substrate and one indenter (Sphere or Plane)
 whose position law is known, and VelocityVerlet -- ``timeStep`` and ``run`` advance with the
 fused device step ``nfx_run_steps`` (a force pass and one node pass per step, indenter position
-computed on the device, replayed from a captured hipGraph of up to 100 steps).  Any other chain
+computed on the device, replayed from a captured hipGraph of 96 steps).  Any other chain
 runs plugin by plugin, exactly like the reference's loop (``Simulation.py:232-237``).
 
 Extensions (keyword arguments):

@@ -1728,6 +1728,25 @@ static nfx_ctx::GraphEntry* find_graph(nfx_ctx* ctx, const nfx_plan& p, const nf
     return nullptr;
 }
 
+// whether a call that holds nblocks whole blocks replays them.  A cell's call of one block captures at the second such
+// call of its plan: the capture takes ten times what one replay gains, and the cell may be stepped once.  Under
+// the caller's own capture the steps are launched one by one
+static bool replays(nfx_ctx* ctx, const nfx_plan& p, const nfx_batch* b, bool hist, int64_t nblocks) {
+    if (nblocks < 1) return false;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (ctx->stream && hipStreamIsCapturing(ctx->stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone) return false;
+    if (b || nblocks > 1 || find_graph(ctx, p, b, hist)) return true;
+    auto& seen = ctx->one_block;
+    for (size_t i = 0; i < seen.size(); ++i)
+        if (seen[i].second == hist && std::memcmp(&seen[i].first, &p, sizeof(nfx_plan)) == 0) {
+            seen.erase(seen.begin() + (std::ptrdiff_t)i);
+            return true;
+        }
+    if ((int)seen.size() >= kMaxGraphs) seen.erase(seen.begin());
+    seen.emplace_back(p, hist);
+    return false;
+}
+
 // capture kGraphBlock steps of the plan (b == NULL) or of the batch; steps read the device step
 // counter ctx->step_dev, so a replay is valid at any step offset
 static int capture_graph(nfx_ctx* ctx, const nfx_plan& p, const nfx_batch* b, bool hist, nfx_ctx::GraphEntry** out) {
@@ -1755,7 +1774,7 @@ static int capture_graph(nfx_ctx* ctx, const nfx_plan& p, const nfx_batch* b, bo
             rc = launch_batch_step(ctx, p, *b, 0, ctx->step_dev, (int32_t)i);
         } else if (node_fused(p)) {
             // launch i of a block is launch k0 + i of its call with k0 even (run_fused starts blocks at
-            // k = 2, 102, ...), so its buffers are those of launch 2 + i
+            // k = 2, 98, ...), so its buffers are those of launch 2 + i
             const int64_t ntiles = (p.T + p.tile_k - 1) / p.tile_k;
             rc = launch_fused(ctx, p, false,
                               fused_io(p, 2 + i, hist ? ctx->tip_rows + i * ntiles : nullptr, 0, ctx->step_dev, (int32_t)i));
@@ -1848,7 +1867,7 @@ static int run_fused(nfx_ctx* c, const nfx_plan& p, int64_t step0, int64_t n, do
     rc = eager(1);
     if (rc) return rc;
     int64_t k = 2;
-    if (use_graph && n - 1 - k >= kGraphBlock) {
+    if (use_graph && replays(c, p, nullptr, tip_hist != nullptr, (n - 1 - k) / kGraphBlock)) {
         const bool hist = tip_hist != nullptr;
         nfx_ctx::GraphEntry* ge = find_graph(c, p, nullptr, hist);
         if (!ge) {
@@ -1883,7 +1902,7 @@ static int run_fused_batch(nfx_ctx* c, const nfx_plan& p, const nfx_batch& b, in
     rc = eager(1);
     if (rc) return rc;
     int64_t k = 2;
-    if (use_graph && n - k >= kGraphBlock) {
+    if (use_graph && replays(c, p, &b, false, (n - k) / kGraphBlock)) {
         nfx_ctx::GraphEntry* ge = find_graph(c, p, &b, false);
         if (!ge) {
             rc = capture_graph(c, p, &b, false, &ge);
@@ -2424,7 +2443,7 @@ int nfx_run_steps(nfx_ctx* c, const nfx_plan* p, int64_t step0, int64_t nsteps, 
     if (rc) return rc;
     int64_t done = 1;
     const int64_t ngraph = nsteps - 1;  // middle steps run while done < ngraph
-    if (use_graph && ngraph - done >= kGraphBlock) {
+    if (use_graph && replays(c, *p, nullptr, tip_hist != nullptr, (ngraph - done) / kGraphBlock)) {
         const int64_t B = kGraphBlock;
         const bool hist = tip_hist != nullptr;
         nfx_ctx::GraphEntry* ge = find_graph(c, *p, nullptr, hist);
@@ -2533,7 +2552,7 @@ int nfx_batch_run_steps(nfx_ctx* c, const nfx_plan* p, const nfx_batch* b, int64
     NFX_REQUIRE(nsteps >= 0, "nsteps < 0");
     if (node_fused(*p) && nsteps >= 2) return run_fused_batch(c, *p, *b, step0, nsteps, use_graph != 0);
     int64_t done = 0;
-    if (use_graph && nsteps >= kGraphBlock) {  // as in nfx_run_steps: whole blocks replay, the rest is eager
+    if (use_graph && replays(c, *p, b, false, nsteps / kGraphBlock)) {  // as in nfx_run_steps: whole blocks replay, the rest is eager
         const int64_t B = kGraphBlock;
         nfx_ctx::GraphEntry* ge = find_graph(c, *p, b, false);
         if (!ge) {
