@@ -197,47 +197,52 @@ __global__ __launch_bounds__(256) void k_gemm_tile(nfx_mlp_gemm_args g) {
     }
 }
 
-// The same product for grids that fill the chip (M, N multiples of 128; one pass over K): a
-// workgroup tile of 128 x 128 staged through LDS, each wave a 64 x 64 sub-tile (4 x 4 MFMA tiles,
-// 16 MFMAs per k-step from 8 LDS fragment reads instead of 4 MFMAs per 4 global reads).  Double
+// Workgroups go to the 8 XCDs in turn: each XCD takes a contiguous range of the output's tiles, so that the tiles of
+// the same rows share the reads of A in its L2
+__device__ __forceinline__ int xcd_tile(int b, int nb) {
+    const int q = nb >> 3, r = nb & 7, x = b & 7;
+    return x * q + (x < r ? x : r) + (b >> 3);
+}
+
+// The same product for grids that fill the chip (M a multiple of 128, N of kTN; one pass over K): a
+// workgroup tile of 128 x kTN staged through LDS, each wave a 64 x 64 sub-tile (4 x 4 MFMA tiles,
+// 16 MFMAs per k-step from 8 LDS fragment reads).  Double
 // buffered: the next k-slice goes global -> registers during the MFMAs and registers -> the other
 // LDS buffer after them, one barrier per k-step.  Rows are padded by 8 BF16 against bank
 // conflicts.  Accumulator layout and epilogue as k_gemm_tile.  Four waves per SIMD (the accumulators
-// then live in VGPRs, 124 of them; the 40 KB of LDS per workgroup fit four workgroups per CU): 13-30 %
-// faster than the three the unbounded allocation gives.
+// then live in VGPRs; the LDS fits them): 13-30 % faster than the three the unbounded allocation gives.
+// The products are bound by what the L2s deliver: the layer of 65 536 x 512 with K = 512 and GELU takes 74.5 us with
+// 128 x 128 tiles in launch order, 66.5 with each XCD's tiles together, 64.3 (0.53 PFLOP/s; 37 us are the epilogue's) with
+// 128 x 256 tiles too, which read a quarter less.  256 x 256 tiles, one workgroup of 16 waves per CU, took 69
 constexpr int kLdsTile = 128, kLdsK = 32, kLdsPitch = kLdsK + 8;
-template <int EPI>
-__global__ __launch_bounds__(256, 4) void k_gemm_lds(nfx_mlp_gemm_args g) {
-    __shared__ __align__(16) __bf16 As[2][kLdsTile * kLdsPitch];
-    __shared__ __align__(16) __bf16 Bs[2][kLdsTile * kLdsPitch];
+template <int EPI, int kTN>
+__global__ __launch_bounds__(2 * kTN, 4) void k_gemm_lds(nfx_mlp_gemm_args g) {
+    constexpr int kThreads = 2 * kTN, kRows = kLdsTile + kTN, kPer = 4 * kRows / kThreads;
+    __shared__ __align__(16) __bf16 S[2][kRows * kLdsPitch];  // the rows of A, then those of B
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
-    const int m0 = blockIdx.y * kLdsTile, n0 = blockIdx.x * kLdsTile;
-    const __bf16* __restrict__ A = static_cast<const __bf16*>(g.A);
-    const __bf16* __restrict__ B = static_cast<const __bf16*>(g.B);
+    const int wm = (wave & 1) * 64, wn = (wave >> 1) * 64;
+    const int tile = xcd_tile((int)(blockIdx.y * gridDim.x + blockIdx.x), (int)(gridDim.x * gridDim.y));
+    const int m0 = tile / (int)gridDim.x * kLdsTile, n0 = tile % (int)gridDim.x * kTN;
     const int r16 = lane & 15, kq = 8 * (lane >> 4);
-    // copy assignment: 128 rows x 4 chunks of 8 BF16 per operand, two chunks per thread
-    int crow[2], ck[2];
+    // copy assignment: 4 chunks of 8 BF16 per row
+    const __bf16* src[kPer];
+    int dst[kPer];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int c = tid + 256 * i;
-        crow[i] = c >> 2;
-        ck[i] = (c & 3) * 8;
+    for (int i = 0; i < kPer; ++i) {
+        const int c = tid + kThreads * i, row = c >> 2, kc = (c & 3) * 8;
+        src[i] = (row < kLdsTile ? static_cast<const __bf16*>(g.A) + (int64_t)(m0 + row) * g.lda
+                                 : static_cast<const __bf16*>(g.B) + (int64_t)(n0 + row - kLdsTile) * g.ldb) +
+                 kc;
+        dst[i] = row * kLdsPitch + kc;
     }
-    bf16x8 ra[2], rb[2];
+    bf16x8 q[kPer];
     auto gload = [&](int k0) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            ra[i] = *reinterpret_cast<const bf16x8*>(A + (int64_t)(m0 + crow[i]) * g.lda + k0 + ck[i]);
-            rb[i] = *reinterpret_cast<const bf16x8*>(B + (int64_t)(n0 + crow[i]) * g.ldb + k0 + ck[i]);
-        }
+        for (int i = 0; i < kPer; ++i) q[i] = *reinterpret_cast<const bf16x8*>(src[i] + k0);
     };
     auto sstore = [&](int buf) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            *reinterpret_cast<bf16x8*>(&As[buf][crow[i] * kLdsPitch + ck[i]]) = ra[i];
-            *reinterpret_cast<bf16x8*>(&Bs[buf][crow[i] * kLdsPitch + ck[i]]) = rb[i];
-        }
+        for (int i = 0; i < kPer; ++i) *reinterpret_cast<bf16x8*>(&S[buf][dst[i]]) = q[i];
     };
     f32x4 acc[4][4];
 #pragma unroll
@@ -254,8 +259,8 @@ __global__ __launch_bounds__(256, 4) void k_gemm_lds(nfx_mlp_gemm_args g) {
         bf16x8 a[4], b[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            a[i] = *reinterpret_cast<const bf16x8*>(&As[buf][(wm + 16 * i + r16) * kLdsPitch + kq]);
-            b[i] = *reinterpret_cast<const bf16x8*>(&Bs[buf][(wn + 16 * i + r16) * kLdsPitch + kq]);
+            a[i] = *reinterpret_cast<const bf16x8*>(&S[buf][(wm + 16 * i + r16) * kLdsPitch + kq]);
+            b[i] = *reinterpret_cast<const bf16x8*>(&S[buf][(kLdsTile + wn + 16 * i + r16) * kLdsPitch + kq]);
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i)
@@ -402,6 +407,17 @@ static void launch_tile(const nfx_mlp_gemm_args& g, int split, hipStream_t s) {
     }
 }
 
+template <int kTN>
+static void launch_lds(const nfx_mlp_gemm_args& g, hipStream_t s) {
+    const dim3 grid(g.N / kTN, g.M / kLdsTile);
+    switch (g.epilogue) {
+        case NFX_MLP_STORE: k_gemm_lds<NFX_MLP_STORE, kTN><<<grid, 2 * kTN, 0, s>>>(g); break;
+        case NFX_MLP_FWD_GELU: k_gemm_lds<NFX_MLP_FWD_GELU, kTN><<<grid, 2 * kTN, 0, s>>>(g); break;
+        case NFX_MLP_BWD_GELU: k_gemm_lds<NFX_MLP_BWD_GELU, kTN><<<grid, 2 * kTN, 0, s>>>(g); break;
+        default: k_gemm_lds<NFX_MLP_ADAM, kTN><<<grid, 2 * kTN, 0, s>>>(g); break;
+    }
+}
+
 }  // namespace nfx
 
 using namespace nfx;
@@ -426,18 +442,15 @@ int nfx_mlp_gemm(nfx_ctx* c, const nfx_mlp_gemm_args* g) {
                 "mlp gemm: split_k %d must be at most 64 and divide K / 32 (K %d)", g->split_k, g->K);
     NFX_REQUIRE(S == 1 || g->workspace, "mlp gemm: split_k > 1 needs a workspace of split_k * M * N floats");
     // the 128 x 128 tiles where they still give a full grid (>= 256 workgroups): less is read per product, but fewer
-    // workgroups hide the latency (K 512, GELU:
-    // 512 tiles 30 us against 34 with the smaller tiles, 128 tiles 22 against 11)
+    // workgroups hide the latency (K 512, GELU: 512 tiles 24 us against 34 with the smaller tiles, 128 tiles 22
+    // against 11)
     const bool lds = S == 1 && g->M % kLdsTile == 0 && g->N % kLdsTile == 0 &&
                      (int64_t)(g->M / kLdsTile) * (g->N / kLdsTile) >= 256;
     if (lds) {
-        const dim3 grid(g->N / kLdsTile, g->M / kLdsTile);
-        switch (g->epilogue) {
-            case NFX_MLP_STORE: k_gemm_lds<NFX_MLP_STORE><<<grid, 256, 0, c->stream>>>(*g); break;
-            case NFX_MLP_FWD_GELU: k_gemm_lds<NFX_MLP_FWD_GELU><<<grid, 256, 0, c->stream>>>(*g); break;
-            case NFX_MLP_BWD_GELU: k_gemm_lds<NFX_MLP_BWD_GELU><<<grid, 256, 0, c->stream>>>(*g); break;
-            default: k_gemm_lds<NFX_MLP_ADAM><<<grid, 256, 0, c->stream>>>(*g); break;
-        }
+        // the wide tiles where two workgroups per CU are left (K 512, GELU, us, wide against 128 x 128: 65 536 x 512
+        // 64.3 / 66.5, 32 768 x 512 35.4 / 37.0, 65 536 x 256 36.4 / 37.8; 24 576 x 512 32.9 / 30.3, 16 384 x 256 21.7 / 19.0)
+        if (g->N % 256 == 0 && (int64_t)(g->M / kLdsTile) * (g->N / 256) >= 512) launch_lds<256>(*g, c->stream);
+        else launch_lds<128>(*g, c->stream);
     } else {
         // k-steps of 64 where they divide a slice; a 32 x 32 tile with k-steps of 32 elsewhere
         if (g->K / S % 64 == 0) launch_tile<64, 32, 64>(*g, S, c->stream);

@@ -35,7 +35,8 @@ def shifted(n, dtype, off):
 # each kind, operands with longer rows, the transposed copy at 8-byte and at 2-byte alignment
 @pytest.mark.parametrize("M,N,K,S,pad,off", [(128, 32, 32, 1, 0, 0), (128, 32, 96, 1, 8, 1), (128, 96, 64, 1, 0, 3),
                                              (384, 64, 192, 1, 24, 0), (256, 64, 96, 3, 0, 2), (128, 160, 448, 7, 8, 0),
-                                             (32768, 128, 64, 1, 0, 1)])
+                                             (32768, 128, 64, 1, 0, 1), (33024, 512, 32, 1, 8, 0),
+                                             (65536, 256, 96, 1, 0, 0)])
 def test_gemm_of_whole_numbers_is_exact(ctx, M, N, K, S, pad, off):
     import torch
 
