@@ -426,14 +426,14 @@ struct NodeStep {
 };
 
 // node n's update (k_node_update's arithmetic, the substrate/indenter/fix choices uniform at run
-// time): x holds u before the step on entry and after it on return; tip receives the node's indenter
-// force when this tile stores the node
+// time): x holds u before the step on entry and after it on return, w the state after it; tip receives the node's
+// indenter force when this tile stores the node (the caller's stores)
 __device__ __forceinline__ void node_step(const NodeStep& s, const ContactConsts& cc, V3 X0, int64_t N, uint32_t n,
-                                          uint32_t dst, uint2 rg, double pos, V3& x, double& tip) {
+                                          uint32_t dst, uint2 rg, double pos, V3& x, V3& w, double& tip) {
     const uint32_t b = rg.x, e = rg.y;
     // before the partials' sum (and X0 with x): behind the contacts' branches these loads were a memory round of their
     // own (steps of a 105 k tetra cell 6.7 -> 6.4 us, of a 0.5 M one 17.5 -> 16.9, of 32 cells of together 1.4 M 32 -> 30)
-    V3 w = mk(s.w[n], s.w[N + n], s.w[2 * N + n]);
+    w = mk(s.w[n], s.w[N + n], s.w[2 * N + n]);
     V3 f = sum_partials8(s.prev_partials, b, e);
     auto xz = [&] { return make_float2(X0.x, X0.z); };
     double tf = 0.0, td = 0.0;
@@ -460,11 +460,7 @@ __device__ __forceinline__ void node_step(const NodeStep& s, const ContactConsts
         x.x = -X0.x;
         x.z = -X0.z;
     }
-    if (dst == b) {
-        s.x_next[n] = x.x; s.x_next[N + n] = x.y; s.x_next[2 * N + n] = x.z;
-        s.w_next[n] = w.x; s.w_next[N + n] = w.y; s.w_next[2 * N + n] = w.z;
-        tip = tf;
-    }
+    if (dst == b) tip = tf;
 }
 
 // ---- force pass, tiled deterministic scatter ---------------------------------------------------
@@ -530,6 +526,12 @@ struct TileArgs {
     // NODE: the previous step's node update (x holds the displacements before it)
     NodeStep ns;
 };
+
+// v is waited for here
+template <class T>
+__device__ __forceinline__ void arrived(T& v) {
+    asm("" : "+v"(v));
+}
 
 // One cell's sample of the batched curves, by one workgroup of any size (<= 512): on the first
 // step of each of the ncurve sample intervals, the indenter force on the cell's nodes at the
@@ -639,7 +641,7 @@ __global__ __launch_bounds__(K, MODEL != NFX_VISCOPLASTIC ? 8 : (STRESS || NODE)
     // cell with flow 16.9 -> 16.2 us, of 32 cells of together 1.4 M 29.7 -> 28.8).  This tetra's 4 corner records (tile-node | rank << 8), as one
     // 8-byte load (whole tiles are stored), and the tile metadata: thread tl owns tile-node tl (MX <= K, checked on
     // the host)
-    const uint64_t cr = ld_g<NT, uint64_t>(uat(reinterpret_cast<const uint64_t*>(a.tile_corners + 4 * K * c), u));
+    uint64_t cr = ld_g<NT, uint64_t>(uat(reinterpret_cast<const uint64_t*>(a.tile_corners + 4 * K * c), u));
     const int64_t j0 = c * (int64_t)MX;
     const bool owner = tl < MX;
     uint32_t nid = 0, dst = 0;
@@ -691,7 +693,7 @@ __global__ __launch_bounds__(K, MODEL != NFX_VISCOPLASTIC ? 8 : (STRESS || NODE)
     }
 
     // this tetra's streaming loads: they overlap the staging phases below
-    float D[9], Sv[MODEL == NFX_VISCOPLASTIC ? 9 : 1], e0 = 0.f, v0 = 0.f, sdm = 0.f;
+    float D[9] = {}, Sv[MODEL == NFX_VISCOPLASTIC ? 9 : 1] = {}, e0 = 0.f, v0 = 0.f, sdm = 0.f;
     if (active) {
         if constexpr (!GEO) {
 #pragma unroll
@@ -712,14 +714,15 @@ __global__ __launch_bounds__(K, MODEL != NFX_VISCOPLASTIC ? 8 : (STRESS || NODE)
         }
     }
     double tip = 0.0;  // NODE: the indenter force on the node this thread stores
+    V3 xn = mk(0.f, 0.f, 0.f), wn = mk(0.f, 0.f, 0.f);  // NODE: the node after the previous step
     if (owner) {
         float ux = a.x[nid], uy = a.x[N + nid], uz = a.x[2 * N + nid];
         V3 X0 = mk(0.f, 0.f, 0.f);
         if constexpr (GEO || NODE) X0 = mk(a.ref[nid], a.ref[N + nid], a.ref[2 * N + nid]);
         if (NODE && tl < M) {  // complete the previous step at this node (padding entries past M are
                                // not nodes of the tile); the forces below see the result
-            V3 xn = mk(ux, uy, uz);
-            node_step(a.ns, cc, X0, N, nid, dst, rg, pos, xn, tip);
+            xn = mk(ux, uy, uz);
+            node_step(a.ns, cc, X0, N, nid, dst, rg, pos, xn, wn, tip);
             ux = xn.x;
             uy = xn.y;
             uz = xn.z;
@@ -738,6 +741,27 @@ __global__ __launch_bounds__(K, MODEL != NFX_VISCOPLASTIC ? 8 : (STRESS || NODE)
 #pragma unroll
             for (int off = 32; off > 0; off >>= 1) tip += __shfl_xor(tip, off);
             if ((tl & 63) == 0) s_tip[tl >> 6] = tip;
+        }
+    }
+    if constexpr (NODE) {
+        // the loads that the law waits for have arrived by now (they are older than the node's); said here, ahead
+        // of the stores: memory instructions are counted in order, and a wait behind the stores would wait for them
+        // (steps of a 105 k tetra cell 6.16 -> 6.02 us, of a 0.5 M one with flow 15.6 -> 15.1)
+        arrived(cr);
+        if constexpr (MODEL == NFX_VISCOPLASTIC) {
+#pragma unroll
+            for (int k = 0; k < (SYM ? 6 : 9); ++k) arrived(Sv[k]);
+            if constexpr (EPS) arrived(e0);
+        }
+        if constexpr (!GEO) {
+#pragma unroll
+            for (int k = 0; k < 9; ++k) arrived(D[k]);
+            arrived(v0);
+        }
+        if (owner && tl < M && dst == rg.x) {  // the node's first tile stores it
+            const NodeStep& s = a.ns;
+            s.x_next[nid] = xn.x; s.x_next[N + nid] = xn.y; s.x_next[2 * N + nid] = xn.z;
+            s.w_next[nid] = wn.x; s.w_next[N + nid] = wn.y; s.w_next[2 * N + nid] = wn.z;
         }
     }
     __syncthreads();
