@@ -50,10 +50,10 @@ def default_stream_nt(tetra):
 # 211k 7.5 / 8.8, 526k 11.7 / 12.5, 878k 16.6 / 16.5; the 3.4M-tetra viscoplastic cell 58 / 50
 NODE_FUSED_MAX_TETRA = 600_000
 # batches hold out longer: their node pass looks each node's cell up, and the curve samples ride in the one launch.
-# Elastic 46k 6.2 / 8.2, 234k 8.1 / 10.0, 733k 17.8 / 18.1, 887k 20.1 / 19.8, 1.4M 24.2 / 25.0, 2.3M 31.9 / 32.5;
-# viscoplastic 46k 6.3 / 8.9, 234k 9.2 / 11.5, 887k 24.4 / 28.5, 1.4M 33.0 / 34.3, 1.9M 41.8 / 42.2, 2.3M 48.6 / 46.8
-# (cells of 10 k to 100 k tetra, 256-tetra tiles, 43 % of the steps with samples from 733k on)
-BATCH_NODE_FUSED_MAX_TETRA = 2_000_000
+# Elastic 46k 6.2 / 8.2, 234k 8.1 / 10.0, 1.4M 23.5 / 24.6, 2.5M 32.0 / 33.5, 3.8M 45.7 / 45.0; viscoplastic 46k 6.3 / 8.9,
+# 234k 9.2 / 11.5, 1.4M 30.1 / 35.1, 2.3M 46.5 / 48.1, 2.5M 49.3 / 51.8, 3.8M 85.3 / 75.1 (cells of 10 k to 100 k tetra,
+# 256-tetra tiles, 43 % of the steps with samples from 1.4M on)
+BATCH_NODE_FUSED_MAX_TETRA = 2_600_000
 
 
 def default_node_fused(tetra):
