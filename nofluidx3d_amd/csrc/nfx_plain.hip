@@ -537,6 +537,7 @@ __device__ __forceinline__ void arrived(T& v) {
 // step of each of the ncurve sample intervals, the indenter force on the cell's nodes at the
 // current positions, summed in FP64 in a fixed order (strided per-thread sums, then lanes and
 // waves in order).  Every exit before the barrier is uniform over the workgroup.
+template <int kDeep>
 __device__ void batch_curve_sample(const float* __restrict__ x, const float* __restrict__ ref, int64_t N,
                                    const uint32_t* __restrict__ cell_node_off, const nfx_cell* __restrict__ cells,
                                    double* curves, int32_t ncurve, int64_t curve_steps, int64_t time, int cell,
@@ -548,18 +549,19 @@ __device__ void batch_curve_sample(const float* __restrict__ x, const float* __r
     const double pos = indenter_pos(cp.tip_start, cp.tip_speed, cp.tip_move_steps, time);
     double s = 0.0;
     const int64_t end = cell_node_off[cell + 1], stride = blockDim.x;
-    // four nodes' loads at a time (the last ones read again past the end, and count nothing there): the pass
-    // is one workgroup's chain of memory rounds
-    for (int64_t n0 = cell_node_off[cell] + threadIdx.x; n0 < end; n0 += 4 * stride) {
-        float xy[4], ry[4];
+    // kDeep nodes' loads at a time (the last ones read again past the end, and count nothing there): the pass is one
+    // workgroup's chain of memory rounds.  Four where the registers hold them; in the two-launch force passes of 7
+    // waves four spill (13 registers in the batch's viscoplastic form, whose launches of 3.8 M tetra took 59 us for 55)
+    for (int64_t n0 = cell_node_off[cell] + threadIdx.x; n0 < end; n0 += kDeep * stride) {
+        float xy[kDeep], ry[kDeep];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < kDeep; ++i) {
             const int64_t n = n0 + i * stride < end ? n0 + i * stride : n0;
             xy[i] = x[N + n];
             ry[i] = ref[N + n];
         }
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < kDeep; ++i) {
             const int64_t n = n0 + i * stride;
             const double y = (double)ry[i] + (double)xy[i];
             if (n >= end) continue;
@@ -601,11 +603,10 @@ enum { META_CELL = 0, META_BATCH = 1, META_BATCH16 = 2 };
 // state is the symmetric deviation Gd (6 planes) instead of Q (9 planes); META: 0 a single
 // cell, 1 a batch, 2 a batch with 16-bit tile-node metadata; NODE: the previous step's node update rides in this pass.  Waves per SIMD: the
 // viscoplastic forms fit 72 VGPRs (7 waves; measured 5 % faster than 6, while the 64-register bound
-// of 8 waves spills and is slower) except with stress outputs or NODE (6), and the symmetric one
-// without epsbar fits 64 (8 waves)
+// of 8 waves spills and is slower) except with stress outputs or NODE (6)
 template <int MODEL, int K, bool GEO, bool STRESS, bool NT = false, bool EPS = true, bool SYM = false,
           int META = META_CELL, bool NODE = false>
-__global__ __launch_bounds__(K, MODEL != NFX_VISCOPLASTIC ? 8 : (STRESS || NODE) ? 6 : (!SYM || EPS) ? 7 : 8) void k_tile_force(TileArgs a, ElasticDev e, VPConst P, float* __restrict__ Sst,
+__global__ __launch_bounds__(K, MODEL != NFX_VISCOPLASTIC ? 8 : (STRESS || NODE) ? 6 : 7) void k_tile_force(TileArgs a, ElasticDev e, VPConst P, float* __restrict__ Sst,
                                                   float* __restrict__ eps, float* __restrict__ vm,
                                                   float* __restrict__ pr) {
     // one thread per tetra of the tile (blockDim.x == K)
@@ -628,7 +629,7 @@ __global__ __launch_bounds__(K, MODEL != NFX_VISCOPLASTIC ? 8 : (STRESS || NODE)
     if (META && blockIdx.x < first_tile) {
         if (blockIdx.x >= (uint32_t)a.curve_blocks) return;
         const int64_t time = a.curve_step_dev ? (*a.curve_step_dev + a.curve_off) : a.curve_step;
-        batch_curve_sample(a.x, a.ref, a.N, a.cell_node_off, a.cells, a.curves, a.ncurve, a.curve_steps, time,
+        batch_curve_sample<NODE ? 4 : 1>(a.x, a.ref, a.N, a.cell_node_off, a.cells, a.curves, a.ncurve, a.curve_steps, time,
                            (int)blockIdx.x, a.curve_ind);
         return;
     }
@@ -693,7 +694,7 @@ __global__ __launch_bounds__(K, MODEL != NFX_VISCOPLASTIC ? 8 : (STRESS || NODE)
     }
 
     // this tetra's streaming loads: they overlap the staging phases below
-    float D[9] = {}, Sv[MODEL == NFX_VISCOPLASTIC ? 9 : 1] = {}, e0 = 0.f, v0 = 0.f, sdm = 0.f;
+    float D[9], Sv[MODEL == NFX_VISCOPLASTIC ? 9 : 1], e0 = 0.f, v0 = 0.f, sdm = 0.f;
     if (active) {
         if constexpr (!GEO) {
 #pragma unroll
@@ -1640,7 +1641,7 @@ __global__ __launch_bounds__(kBlock) void k_batch_curves(const float* __restrict
                                                          int32_t ncurve, int64_t curve_steps, int64_t step,
                                                          const int64_t* step_dev, int32_t step_off) {
     const int64_t time = step_dev ? (*step_dev + step_off) : step;
-    batch_curve_sample(x, ref, N, cell_node_off, cells, curves, ncurve, curve_steps, time, blockIdx.x, IND);
+    batch_curve_sample<4>(x, ref, N, cell_node_off, cells, curves, ncurve, curve_steps, time, blockIdx.x, IND);
 }
 
 static int validate_batch(const nfx_plan* p, const nfx_batch* b) {
