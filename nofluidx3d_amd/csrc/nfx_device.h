@@ -330,20 +330,6 @@ __device__ __forceinline__ Corners cofactor_forces_r(const S6& sig, V3 r1, V3 r2
     return cofactor_forces(sig, Cof3{cross(r2, r3), cross(r3, r1), cross(r1, r2)}, scale);
 }
 
-// f_k = M (s d_k) for rows d_k of D, f0 = -(f1 + f2 + f3)
-__device__ __forceinline__ Corners row_forces(const M9& M, const float* D, float s) {
-    Corners o;
-    V3* f[3] = {&o.f1, &o.f2, &o.f3};
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        const V3 d = mk(D[3 * k + 0] * s, D[3 * k + 1] * s, D[3 * k + 2] * s);
-        *f[k] = mk(M.m[0][0] * d.x + M.m[0][1] * d.y + M.m[0][2] * d.z, M.m[1][0] * d.x + M.m[1][1] * d.y + M.m[1][2] * d.z,
-                   M.m[2][0] * d.x + M.m[2][1] * d.y + M.m[2][2] * d.z);
-    }
-    o.f0 = (o.f1 + o.f2 + o.f3) * -1.0f;
-    return o;
-}
-
 // ---- the material frame ------------------------------------------------------------------------
 // The laws below are isotropic, so sigma cof(F) = J F (F^-1 sigma F^-T), and F^-1 B^n F^-T is a product
 // of the symmetric tensors C = F^T F and its inverse (times I + Gd for an elastic Be): the stress is
@@ -391,14 +377,16 @@ __device__ __forceinline__ Corners material_forces(const S6& S, const M9& H, con
 
 // Mooney-Rivlin / Neo-Hookean branch of tetra.cl:115-168: J = det F (tetra.cl:132 computes
 // det(r) / (6 V0), the same number), rows -V0 J r^-1 sigma = -(1/6) sigma cof(F) (6 V0 d_k).
-// Neo-Hookean (uniform branch): B F^-T = F turns sigma cof(F) into a J F - beta cof(F), beta = a tr B / 3 -
-// kappa (J - 1), with cof(F) = I + i1 I - H^T + cof(H): no stress tensor at all.  Mooney-Rivlin: the material
-// stress a combination of Kd, Cd and I.  About 37 and 25 VALU instructions per tetra less than through the
-// spatial stress; with the tile lists in run-length order the step of a 2.2 M tetra cell takes 26.4-27.6 us
-// (Neo-Hookean, 29.4-30.1 before) and 28.0-28.9 us (Mooney-Rivlin, 29.6-30.6); alone 1.7 % and nothing: LDS
-// and VALU bound the pass together.
+// Neo-Hookean (uniform branch): the stress, then the edge cofactors.  Formed without the stress, as J F less a multiple
+// of cof(F), the rotation in H is rounded twice before it cancels and J F and cof(F) cancel under compression: 3 to 80
+// times the error at rotations of 0.01 to 0.3 with little strain, twice at stretches of 0.5 to 0.6.
+// Mooney-Rivlin: the material stress, a combination of Kd, Cd and I.
 __device__ __forceinline__ Corners mr_tetra(const M9& H, const float* D, float v0, float mu1, float mu2,
                                             float kappa) {
+    if (mu2 == 0.0f) {
+        const S6 sig = mr_stress(cauchy_green_m1(H), det_ipH_m1(H), mu1, mu2, kappa);
+        return cofactor_forces(sig, edge_cofactors(cof_ipH(H), D, 6.0f * v0), -1.0f / 6.0f);
+    }
     const V3 h0 = mk(H.m[0][0], H.m[0][1], H.m[0][2]), h1 = mk(H.m[1][0], H.m[1][1], H.m[1][2]),
              h2 = mk(H.m[2][0], H.m[2][1], H.m[2][2]);
     const V3 q0 = cross(h1, h2), q1 = cross(h2, h0), q2 = cross(h0, h1);  // rows of cof(H)
@@ -409,22 +397,6 @@ __device__ __forceinline__ Corners mr_tetra(const M9& H, const float* D, float v
     const float t2 = t * t, t5 = t2 * t2 * t;
     const float a = mu1 * t5, vol = kappa * Jm1;
     constexpr float sc = -1.0f / 6.0f;
-    if (mu2 == 0.0f) {
-        const float d3 = (2.0f * i1 + (dot(h0, h0) + dot(h1, h1) + dot(h2, h2))) * (1.0f / 3.0f);  // tr(B - I) / 3
-        const float beta = a + (a * d3 - vol);
-        const float c0 = sc * ((a * (Jm1 - d3) + vol) - beta * i1), ch = sc * (a * J), ct = sc * beta;
-        M9 P;
-        P.m[0][0] = ch * h0.x + (ct * (h0.x - q0.x) + c0);
-        P.m[0][1] = ch * h0.y + ct * (h1.x - q0.y);
-        P.m[0][2] = ch * h0.z + ct * (h2.x - q0.z);
-        P.m[1][0] = ch * h1.x + ct * (h0.y - q1.x);
-        P.m[1][1] = ch * h1.y + (ct * (h1.y - q1.y) + c0);
-        P.m[1][2] = ch * h1.z + ct * (h2.y - q1.z);
-        P.m[2][0] = ch * h2.x + ct * (h0.z - q2.x);
-        P.m[2][1] = ch * h2.y + ct * (h1.z - q2.y);
-        P.m[2][2] = ch * h2.z + (ct * (h2.z - q2.z) + c0);
-        return row_forces(P, D, 6.0f * v0);
-    }
     const MaterialFrame f = material_frame(H);
     const S6 K = material_k(f, f.c2 + f.c3);
     const float k = mu2 * t5 * t2, ak = a + k;
