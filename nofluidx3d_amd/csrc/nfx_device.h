@@ -330,81 +330,17 @@ __device__ __forceinline__ Corners cofactor_forces_r(const S6& sig, V3 r1, V3 r2
     return cofactor_forces(sig, Cof3{cross(r2, r3), cross(r3, r1), cross(r1, r2)}, scale);
 }
 
-// ---- the material frame ------------------------------------------------------------------------
-// The laws below are isotropic, so sigma cof(F) = J F (F^-1 sigma F^-T), and F^-1 B^n F^-T is a product
-// of the symmetric tensors C = F^T F and its inverse (times I + Gd for an elastic Be): the stress is
-// formed there and each corner force is F times it times a reference edge normal, without the spatial
-// stress and the cofactors of F.  Cd = C - I and Kd = I - C^-1 come out of H without cancellation
-// (Kd = (Cd - adj Cd + (c2 + c3) I) / J^2 with the principal invariants c1, c2, c3 of Cd).
-struct MaterialFrame {
-    S6 Cd;             // C - I = H + H^T + H^T H
-    S6 A;              // adj Cd
-    float c1, c2, c3;  // J^2 = det C = 1 + c1 + c2 + c3
-};
-__device__ __forceinline__ MaterialFrame material_frame(const M9& H) {
-    MaterialFrame f;
-    const V3 h0 = mk(H.m[0][0], H.m[1][0], H.m[2][0]), h1 = mk(H.m[0][1], H.m[1][1], H.m[2][1]),
-             h2 = mk(H.m[0][2], H.m[1][2], H.m[2][2]);  // columns of H
-    const S6 C{2.0f * h0.x + dot(h0, h0), 2.0f * h1.y + dot(h1, h1), 2.0f * h2.z + dot(h2, h2),
-               (h1.x + h0.y) + dot(h0, h1), (h2.y + h1.z) + dot(h1, h2), (h2.x + h0.z) + dot(h0, h2)};
-    f.Cd = C;
-    f.A = S6{C.yy * C.zz - C.yz * C.yz, C.xx * C.zz - C.xz * C.xz, C.xx * C.yy - C.xy * C.xy,
-             C.xz * C.yz - C.xy * C.zz, C.xy * C.xz - C.xx * C.yz, C.xy * C.yz - C.yy * C.xz};
-    f.c1 = C.xx + C.yy + C.zz;
-    f.c2 = f.A.xx + f.A.yy + f.A.zz;
-    f.c3 = C.xx * f.A.xx + C.xy * f.A.xy + C.xz * f.A.xz;
-    return f;
-}
-// J^2 Kd
-__device__ __forceinline__ S6 material_k(const MaterialFrame& f, float c23) {
-    return S6{f.Cd.xx - f.A.xx + c23, f.Cd.yy - f.A.yy + c23, f.Cd.zz - f.A.zz + c23,
-              f.Cd.xy - f.A.xy, f.Cd.yz - f.A.yz, f.Cd.xz - f.A.xz};
-}
-// the forces of a material stress S: f_k = F (S (s d_k))
-__device__ __forceinline__ Corners material_forces(const S6& S, const M9& H, const float* D, float s) {
-    Corners o;
-    V3* f[3] = {&o.f1, &o.f2, &o.f3};
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        const V3 w = smul(S, mk(D[3 * k + 0] * s, D[3 * k + 1] * s, D[3 * k + 2] * s));
-        *f[k] = mk(w.x + (H.m[0][0] * w.x + H.m[0][1] * w.y + H.m[0][2] * w.z),
-                   w.y + (H.m[1][0] * w.x + H.m[1][1] * w.y + H.m[1][2] * w.z),
-                   w.z + (H.m[2][0] * w.x + H.m[2][1] * w.y + H.m[2][2] * w.z));
-    }
-    o.f0 = (o.f1 + o.f2 + o.f3) * -1.0f;
-    return o;
-}
-
 // Mooney-Rivlin / Neo-Hookean branch of tetra.cl:115-168: J = det F (tetra.cl:132 computes
-// det(r) / (6 V0), the same number), rows -V0 J r^-1 sigma = -(1/6) sigma cof(F) (6 V0 d_k).
-// Neo-Hookean (uniform branch): the stress, then the edge cofactors.  Formed without the stress, as J F less a multiple
-// of cof(F), the rotation in H is rounded twice before it cancels and J F and cof(F) cancel under compression: 3 to 80
-// times the error at rotations of 0.01 to 0.3 with little strain, twice at stretches of 0.5 to 0.6.
-// Mooney-Rivlin: the material stress, a combination of Kd, Cd and I.
+// det(r) / (6 V0), the same number), rows -V0 J r^-1 sigma = -(1/6) sigma c_k.
+// Forms without the spatial stress take fewer instructions and round worse.  Neo-Hookean as J F less a multiple of
+// cof(F): the rotation in H is rounded twice before it cancels, and the two terms cancel under compression (3 to 80 times
+// the error at rotations of 0.01 to 0.3 with little strain, twice at stretches of 0.5 to 0.6).  Mooney-Rivlin through
+// C - I and I - C^-1 = (.. - adj(C - I) ..) / J^2: the square of the conditioning (1.4 times the error at strains of 0.5, 3 to 8
+// times at stretches of 0.4 to 0.7).
 __device__ __forceinline__ Corners mr_tetra(const M9& H, const float* D, float v0, float mu1, float mu2,
                                             float kappa) {
-    if (mu2 == 0.0f) {
-        const S6 sig = mr_stress(cauchy_green_m1(H), det_ipH_m1(H), mu1, mu2, kappa);
-        return cofactor_forces(sig, edge_cofactors(cof_ipH(H), D, 6.0f * v0), -1.0f / 6.0f);
-    }
-    const V3 h0 = mk(H.m[0][0], H.m[0][1], H.m[0][2]), h1 = mk(H.m[1][0], H.m[1][1], H.m[1][2]),
-             h2 = mk(H.m[2][0], H.m[2][1], H.m[2][2]);
-    const V3 q0 = cross(h1, h2), q1 = cross(h2, h0), q2 = cross(h0, h1);  // rows of cof(H)
-    const float i1 = h0.x + h1.y + h2.z;
-    const float Jm1 = i1 + ((q0.x + q1.y + q2.z) + dot(h0, q0));
-    const float J = 1.0f + Jm1;
-    const float t = fexp2(flog2(J) * (-1.0f / 3.0f));
-    const float t2 = t * t, t5 = t2 * t2 * t;
-    const float a = mu1 * t5, vol = kappa * Jm1;
-    constexpr float sc = -1.0f / 6.0f;
-    const MaterialFrame f = material_frame(H);
-    const S6 K = material_k(f, f.c2 + f.c3);
-    const float k = mu2 * t5 * t2, ak = a + k;
-    const float g = vol - (ak * f.c1 + 2.0f * k * f.c2) * (1.0f / 3.0f);
-    const float cj = sc * J, ck = cj * ((ak + (k + k * f.c1)) - g) * frcp(J * J), cc = -cj * k, ci = cj * g;
-    const S6 S{ck * K.xx + (cc * f.Cd.xx + ci), ck * K.yy + (cc * f.Cd.yy + ci), ck * K.zz + (cc * f.Cd.zz + ci),
-               ck * K.xy + cc * f.Cd.xy, ck * K.yz + cc * f.Cd.yz, ck * K.xz + cc * f.Cd.xz};
-    return material_forces(S, H, D, 6.0f * v0);
+    const S6 sig = mr_stress(cauchy_green_m1(H), det_ipH_m1(H), mu1, mu2, kappa);
+    return cofactor_forces(sig, edge_cofactors(cof_ipH(H), D, 6.0f * v0), -1.0f / 6.0f);
 }
 
 // rows f1..f3 of  -V0 mu * D * M * F^T  (tetra.cl:93 and :114 share this shape), M symmetric or not

@@ -67,6 +67,7 @@ def spatial_form(H, mu1, mu2, kappa, rng=None):
 @pytest.mark.parametrize("ratio,kind,size", [
     (1.0, "rotation", 0.01), (1.0, "rotation", 0.03), (1.0, "strain", 0.001), (1.0, "strain", 0.1),
     (1.0, "stretch", 0.5), (1.0, "stretch", 0.9),
+    (0.75, "rotation", 0.03), (0.75, "strain", 0.1), (0.75, "stretch", 0.5), (0.25, "stretch", 0.6), (0.25, "stretch", 0.9),
 ])
 def test_law_rounds_no_more_than_its_spatial_form(ctx, nu, ratio, kind, size):  # noqa: F811
     import torch
