@@ -218,15 +218,17 @@ __device__ __forceinline__ float det_dm(const float* D) {
 struct Cof3 {
     V3 c1, c2, c3;
 };
-// c_k = C (s d_k) for rows d_k of D (D = Dm^-1 with s = det Dm, or D = G with s = 1)
+// c_k = C (s d_k) for rows d_k of D (D = Dm^-1 with s = det Dm, or D = G with s = 1).  The fused products are written
+// out: left to the compiler, which of a row's products is rounded by itself differed between the kernels of the two step
+// forms on streamed shapes, whose steps then differed in the last bits
 __device__ __forceinline__ Cof3 edge_cofactors(const M9& C, const float* D, float s) {
     Cof3 o;
     V3* c[3] = {&o.c1, &o.c2, &o.c3};
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
         const V3 d = mk(D[3 * k + 0] * s, D[3 * k + 1] * s, D[3 * k + 2] * s);
-        *c[k] = mk(C.m[0][0] * d.x + C.m[0][1] * d.y + C.m[0][2] * d.z, C.m[1][0] * d.x + C.m[1][1] * d.y + C.m[1][2] * d.z,
-                   C.m[2][0] * d.x + C.m[2][1] * d.y + C.m[2][2] * d.z);
+        auto row = [&](const float* r) { return __builtin_fmaf(r[2], d.z, __builtin_fmaf(r[0], d.x, r[1] * d.y)); };
+        *c[k] = mk(row(C.m[0]), row(C.m[1]), row(C.m[2]));
     }
     return o;
 }

@@ -26,3 +26,18 @@ def test_ordered_tile_lists_change_no_bit(ctx, tile_k, material):  # noqa: F811
         out.append((host(sim.displacement, np.float32), host(sim.interactions[-1].velocityB, np.float32)))
     assert np.abs(out[0][0]).max() > 0
     assert all(np.array_equal(a, b) for a, b in zip(*out))
+
+
+@pytest.mark.parametrize("geo", [True, False])
+@pytest.mark.parametrize("material", ["NH", "MR", "VP"])
+def test_one_launch_steps_match_two_launch_steps(ctx, material, geo):  # noqa: F811
+    """with the shape from the reference positions and with the streamed shape"""
+    out = []
+    for fuse in (True, False):
+        sim = build_sim(scatter="tiled", material=material)
+        sim.tile_k, sim.shape_from_ref, sim.fuse_node_pass = 128, geo, fuse
+        assert bool(sim.plan().disp_b) == fuse
+        sim.advance(120)
+        out.append((host(sim.displacement, np.float32), host(sim.interactions[-1].velocityB, np.float32)))
+    assert np.abs(out[0][0]).max() > 0
+    assert all(np.array_equal(a, b) for a, b in zip(*out))
