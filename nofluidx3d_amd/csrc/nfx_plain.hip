@@ -1633,13 +1633,15 @@ __global__ __launch_bounds__(kBlock) void k_batch_node(BatchNodeArgs a, int64_t 
 }
 
 // One workgroup per cell: on a sampling step, the cell's indenter force (Simulation.py:198-212 in
-// simulation units) from the positions at the start of the step, summed in FP64 in a fixed order.
+// simulation units) from the positions at the start of the step, summed in FP64 in a fixed order.  The order depends on
+// the workgroup's size: tile_k threads, as the samples inside a force pass have, so that a curve does not depend on how
+// its steps are split into calls.
 template <int IND>
-__global__ __launch_bounds__(kBlock) void k_batch_curves(const float* __restrict__ x, const float* __restrict__ ref,
-                                                         int64_t N, const uint32_t* __restrict__ cell_node_off,
-                                                         const nfx_cell* __restrict__ cells, double* curves,
-                                                         int32_t ncurve, int64_t curve_steps, int64_t step,
-                                                         const int64_t* step_dev, int32_t step_off) {
+__global__ __launch_bounds__(512) void k_batch_curves(const float* __restrict__ x, const float* __restrict__ ref,
+                                                      int64_t N, const uint32_t* __restrict__ cell_node_off,
+                                                      const nfx_cell* __restrict__ cells, double* curves,
+                                                      int32_t ncurve, int64_t curve_steps, int64_t step,
+                                                      const int64_t* step_dev, int32_t step_off) {
     const int64_t time = step_dev ? (*step_dev + step_off) : step;
     batch_curve_sample<4>(x, ref, N, cell_node_off, cells, curves, ncurve, curve_steps, time, blockIdx.x, IND);
 }
@@ -1672,10 +1674,10 @@ static void launch_batch_node_sub(nfx_ctx* ctx, const nfx_plan& p, const BatchNo
 static int launch_batch_curves(nfx_ctx* ctx, const nfx_plan& p, const nfx_batch& b, const float* x, int64_t step,
                                const int64_t* sd, int32_t off) {
     if (p.indenter == NFX_INDENTER_SPHERE)
-        k_batch_curves<1><<<b.ncells, kBlock, 0, ctx->stream>>>(x, p.ref, p.N, b.cell_node_off, b.cells, b.curves,
+        k_batch_curves<1><<<b.ncells, p.tile_k, 0, ctx->stream>>>(x, p.ref, p.N, b.cell_node_off, b.cells, b.curves,
                                                                 b.ncurve, b.curve_steps, step, sd, off);
     else
-        k_batch_curves<2><<<b.ncells, kBlock, 0, ctx->stream>>>(x, p.ref, p.N, b.cell_node_off, b.cells, b.curves,
+        k_batch_curves<2><<<b.ncells, p.tile_k, 0, ctx->stream>>>(x, p.ref, p.N, b.cell_node_off, b.cells, b.curves,
                                                                 b.ncurve, b.curve_steps, step, sd, off);
     NFX_CHECK_LAUNCH();
     return NFX_OK;

@@ -56,3 +56,27 @@ def test_one_launch_steps_match_two_launch_steps(ctx, monkeypatch, viscous, kw):
     assert float(two[2].abs().max()) > 0.0 and bool(torch.isfinite(two[0]).all())
     for s, t in zip(one, two):
         assert np.array_equal(s.cpu().numpy(), t.cpu().numpy())
+
+
+@pytest.mark.parametrize("tile_k", [128, 256, 512])
+def test_curves_do_not_depend_on_the_split_into_calls(ctx, monkeypatch, tile_k):
+    """every step is a sample, so every call ends on one, with many nodes in contact: the sum's order is the same in
+    a call's last step as inside a call, in both step forms"""
+    from nofluidx3d_amd import autotune
+    from nofluidx3d_amd.batch import BatchSimulation, CellSpec, make_meshes
+
+    specs = [CellSpec(3.0, 0.3, 3200 + i, 500.0, 0.4, None, 5.0, 3.0, indent_frac=0.5) for i in range(2)]
+    meshes = make_meshes(specs, workers=1, cache=None)
+
+    def run(limit, calls):
+        monkeypatch.setattr(autotune, "BATCH_NODE_FUSED_MAX_TETRA", limit)
+        b = BatchSimulation(specs, meshes, steps=400, ncurve=400, tile_k=tile_k)
+        assert bool(b.plan.disp_b) == (limit > 0)
+        for n in calls:
+            b.advance(n)
+        return b.curves_sim()
+
+    whole = run(0, [400])
+    assert (whole[:, 200:] > 0).all()
+    for limit, calls in ((0, [7] * 57 + [1]), (10 ** 9, [400]), (10 ** 9, [7] * 57 + [1]), (10 ** 9, [2] * 200)):
+        assert np.array_equal(run(limit, calls), whole)
