@@ -527,10 +527,11 @@ struct TileArgs {
     NodeStep ns;
 };
 
-// v is waited for here
-template <class T>
-__device__ __forceinline__ void arrived(T& v) {
-    asm("" : "+v"(v));
+// Every load issued so far has arrived, and no store behind this moves ahead of it.  A wait of its own and not a use of the
+// loaded values: those are indeterminate in lanes that loaded nothing
+__device__ __forceinline__ void wait_for_loads() {
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // gfx9 encoding: vmcnt 0, expcnt and lgkmcnt any
+    asm volatile("" : : : "memory");
 }
 
 // One cell's sample of the batched curves, by one workgroup of any size (<= 512): on the first
@@ -748,17 +749,7 @@ __global__ __launch_bounds__(K, MODEL != NFX_VISCOPLASTIC ? 8 : (STRESS || NODE)
         // the loads that the law waits for have arrived by now (they are older than the node's); said here, ahead
         // of the stores: memory instructions are counted in order, and a wait behind the stores would wait for them
         // (steps of a 105 k tetra cell 6.16 -> 6.02 us, of a 0.5 M one with flow 15.6 -> 15.1)
-        arrived(cr);
-        if constexpr (MODEL == NFX_VISCOPLASTIC) {
-#pragma unroll
-            for (int k = 0; k < (SYM ? 6 : 9); ++k) arrived(Sv[k]);
-            if constexpr (EPS) arrived(e0);
-        }
-        if constexpr (!GEO) {
-#pragma unroll
-            for (int k = 0; k < 9; ++k) arrived(D[k]);
-            arrived(v0);
-        }
+        wait_for_loads();
         if (owner && tl < M && dst == rg.x) {  // the node's first tile stores it
             const NodeStep& s = a.ns;
             s.x_next[nid] = xn.x; s.x_next[N + nid] = xn.y; s.x_next[2 * N + nid] = xn.z;
