@@ -604,10 +604,12 @@ enum { META_CELL = 0, META_BATCH = 1, META_BATCH16 = 2 };
 // state is the symmetric deviation Gd (6 planes) instead of Q (9 planes); META: 0 a single
 // cell, 1 a batch, 2 a batch with 16-bit tile-node metadata; NODE: the previous step's node update rides in this pass.  Waves per SIMD: the
 // viscoplastic forms fit 72 VGPRs (7 waves; measured 5 % faster than 6, while the 64-register bound
-// of 8 waves spills and is slower) except with stress outputs or NODE (6)
+// of 8 waves spills and is slower) except with stress outputs or NODE (6).  A single cell's compact state (SYM without
+// EPS) takes 8, at 2 to 4 spilled registers: step of a 3.4 M tetra cell with tiles of 512 49.9 us at 7, 45.9 at 8 (tiles of 256
+// 44.9 and 45.2), of a 0.5 M one 12.5 and 11.65 (11.9 and 11.8).  The batches' form spills more there and takes 7
 template <int MODEL, int K, bool GEO, bool STRESS, bool NT = false, bool EPS = true, bool SYM = false,
           int META = META_CELL, bool NODE = false>
-__global__ __launch_bounds__(K, MODEL != NFX_VISCOPLASTIC ? 8 : (STRESS || NODE) ? 6 : 7) void k_tile_force(TileArgs a, ElasticDev e, VPConst P, float* __restrict__ Sst,
+__global__ __launch_bounds__(K, MODEL != NFX_VISCOPLASTIC ? 8 : (STRESS || NODE) ? 6 : (SYM && !EPS && META == META_CELL) ? 8 : 7) void k_tile_force(TileArgs a, ElasticDev e, VPConst P, float* __restrict__ Sst,
                                                   float* __restrict__ eps, float* __restrict__ vm,
                                                   float* __restrict__ pr) {
     // one thread per tetra of the tile (blockDim.x == K)
