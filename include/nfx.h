@@ -214,7 +214,10 @@ typedef struct {
 int nfx_device_count(int* count);                        /* openCL.py:20-28 device walk */
 int nfx_init(int device_id, void* stream, nfx_ctx** ctx); /* openCL.py:17-34 initializeOpenCLObjects;
                                                              stream: hipStream_t to use, NFX_STREAM_DEFAULT, or
-                                                             NULL for a library-owned default-priority stream */
+                                                             NULL for a library-owned default-priority stream.
+                                                             Makes device_id the calling thread's current device;
+                                                             calls on ctx work on it whatever device is current then,
+                                                             and leave that one current */
 int nfx_destroy(nfx_ctx* ctx);
 int nfx_stream_sync(nfx_ctx* ctx); /* getCommandQueue().finish(), Simulation.py:266 */
 const char* nfx_last_error(void);

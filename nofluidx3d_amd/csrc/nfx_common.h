@@ -88,3 +88,34 @@ struct nfx_ctx {
     uint64_t graph_clock = 0;
     int64_t captures = 0;  // graphs captured so far (nfx_graph_captures)
 };
+
+namespace nfx {
+
+// The calling thread's current device is the context's while an entry point runs, and its own again afterwards: a launch on
+// the default stream and an allocation go to the current device, which is another one after the caller's hipSetDevice or in
+// a thread that never chose one
+class DeviceScope {
+public:
+    explicit DeviceScope(const nfx_ctx* c) {
+        if (!c || (err_ = hipGetDevice(&before_)) != hipSuccess || before_ == c->device) return;
+        err_ = hipSetDevice(c->device);
+        switched_ = err_ == hipSuccess;
+    }
+    ~DeviceScope() {
+        if (switched_) (void)hipSetDevice(before_);
+    }
+    DeviceScope(const DeviceScope&) = delete;
+    DeviceScope& operator=(const DeviceScope&) = delete;
+    hipError_t error() const { return err_; }
+
+private:
+    int before_ = -1;
+    hipError_t err_ = hipSuccess;
+    bool switched_ = false;
+};
+
+}  // namespace nfx
+
+#define NFX_ON_DEVICE(ctx)                        \
+    const ::nfx::DeviceScope device_scope_(ctx);  \
+    NFX_HIP(device_scope_.error())

@@ -358,6 +358,7 @@ using namespace nfx;
 extern "C" {
 
 int nfx_round_tip_force(nfx_ctx* c, float* force, const float* points, int64_t N, double radius, double sphere_pos) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(c && force && points, "NULL argument");
     if (int rc = check_n(N, "node")) return rc;
     k_round_tip<<<nb_of(N), kB, 0, c->stream>>>(force, points, N, (float)radius, (float)sphere_pos);
@@ -367,6 +368,7 @@ int nfx_round_tip_force(nfx_ctx* c, float* force, const float* points, int64_t N
 
 int nfx_adhesive_plane_force(nfx_ctx* c, float* force, const float* points, int64_t N, double wall_pos,
                              double adhesion, double distance, const int32_t* on_surface) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(c && force && points && on_surface, "NULL argument");
     if (int rc = check_n(N, "node")) return rc;
     const double sigma = std::pow(0.5, 1.0 / 6.0) * distance;  // InteractionAdhesivePlane.cl:6
@@ -377,6 +379,7 @@ int nfx_adhesive_plane_force(nfx_ctx* c, float* force, const float* points, int6
 }
 
 int nfx_point_zero_force(nfx_ctx* c, float* force, const float* points, int64_t N, double k) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(c && force && points, "NULL argument");
     if (int rc = check_n(N, "node")) return rc;
     k_point_zero<<<nb_of(N), kB, 0, c->stream>>>(force, points, N, (float)k);
@@ -385,6 +388,7 @@ int nfx_point_zero_force(nfx_ctx* c, float* force, const float* points, int64_t 
 }
 
 int nfx_center_of_mass(nfx_ctx* c, const float* points, int64_t N, double* com) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(c && points && com, "NULL argument");
     if (int rc = check_n(N, "node")) return rc;
     const int nb = (int)std::min<int64_t>(nb_of(N), kMaxReduceBlocks);
@@ -396,6 +400,7 @@ int nfx_center_of_mass(nfx_ctx* c, const float* points, int64_t N, double* com) 
 }
 
 int nfx_com_force(nfx_ctx* c, float* force, int64_t N, double k, const double* com) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(c && force && com, "NULL argument");
     if (int rc = check_n(N, "node")) return rc;
     k_com_force<<<nb_of(N), kB, 0, c->stream>>>(force, N, (float)k, com);
@@ -404,6 +409,7 @@ int nfx_com_force(nfx_ctx* c, float* force, int64_t N, double k, const double* c
 }
 
 int nfx_over_damped(nfx_ctx* c, float* points, float* force, int64_t N, int32_t point3fix) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(c && points && force, "NULL argument");
     if (int rc = check_n(N, "node")) return rc;
     k_over_damped<<<nb_of(N), kB, 0, c->stream>>>(points, force, N, point3fix);
@@ -413,6 +419,7 @@ int nfx_over_damped(nfx_ctx* c, float* points, float* force, int64_t N, int32_t 
 
 int nfx_velocity_verlet2(nfx_ctx* c, float* points, float* vel, float* force, float* fold, const float* masses,
                          int64_t N, double damping) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(c && points && vel && force && fold && masses, "NULL argument");
     if (int rc = check_n(N, "node")) return rc;
     k_vv2<<<nb_of(N), kB, 0, c->stream>>>(points, vel, force, fold, masses, N, (float)damping);
@@ -423,6 +430,7 @@ int nfx_velocity_verlet2(nfx_ctx* c, float* points, float* vel, float* force, fl
 int nfx_volume_integral_force(nfx_ctx* c, int32_t tip_shape, const float* points, const uint32_t* tetras, int64_t N,
                               int64_t T, double radius, double half_angle, double tip_x, double tip_y, double tip_z,
                               double k, float* force, float* corners) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(c && points && tetras && (force || corners), "NULL argument");
     if (int rc = check_n(N, "node")) return rc;
     if (int rc = check_n(T, "tetra")) return rc;
@@ -440,6 +448,7 @@ int nfx_volume_integral_force(nfx_ctx* c, int32_t tip_shape, const float* points
 int nfx_linear_viscoelastic_force(nfx_ctx* c, const nfx_viscoelastic* p, const float* points, const uint32_t* tetras,
                                   const float* dminv, int64_t N, int64_t T, float* dev_old, float* transient,
                                   float* von_mises, float* pressure, float* force, float* corners) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(c && p && points && tetras && dminv && dev_old && (force || corners), "NULL argument");
     NFX_REQUIRE(p->nterms >= 0 && p->nterms <= 8, "viscoelastic terms %d outside 0..8", p->nterms);
     NFX_REQUIRE(p->nterms == 0 || transient, "NULL transient stresses");
@@ -471,6 +480,7 @@ int nfx_linear_viscoelastic_force(nfx_ctx* c, const nfx_viscoelastic* p, const f
 
 int nfx_adhesive_plane_surface_force(nfx_ctx* c, float* force, const float* points, const uint32_t* triangles,
                                      int64_t N, int64_t NT, double wall_pos, double adhesion, double distance) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(c && force && points && triangles, "NULL argument");
     if (int rc = check_n(N, "node")) return rc;
     if (int rc = check_n(NT, "triangle")) return rc;
@@ -484,6 +494,7 @@ int nfx_adhesive_plane_surface_force(nfx_ctx* c, float* force, const float* poin
 int nfx_hard_adhesive_plane_surface_force(nfx_ctx* c, float* force, const float* points, const uint32_t* triangles,
                                           int64_t N, int64_t NT, double wall_pos, double adhesion,
                                           double force_const) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(c && force && points && triangles, "NULL argument");
     if (int rc = check_n(N, "node")) return rc;
     if (int rc = check_n(NT, "triangle")) return rc;

@@ -425,6 +425,7 @@ using namespace nfx;
 extern "C" {
 
 int nfx_mlp_gemm(nfx_ctx* c, const nfx_mlp_gemm_args* g) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(c && g, "NULL argument");
     NFX_REQUIRE(g->M > 0 && g->N > 0 && g->K > 0 && g->M % 128 == 0 && g->N % 32 == 0 && g->K % 32 == 0,
                 "mlp gemm: M must be a multiple of 128, N and K of 32 (got %d %d %d)", g->M, g->N, g->K);
@@ -472,6 +473,7 @@ int nfx_mlp_gemm(nfx_ctx* c, const nfx_mlp_gemm_args* g) {
 
 int nfx_mlp_mse(nfx_ctx* c, const float* Y, const float* target, const float* row_weight, int32_t M, int32_t N,
                 void* dZ, void* dZT, double* loss_sum) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(c && Y && target && dZ && dZT && loss_sum, "NULL argument");
     NFX_REQUIRE(M > 0 && N > 0 && M % 32 == 0 && N % 32 == 0, "mlp mse: M and N must be multiples of 32 (got %d %d)",
                 M, N);
@@ -486,6 +488,7 @@ int nfx_mlp_mse(nfx_ctx* c, const float* Y, const float* target, const float* ro
 
 int nfx_mlp_bias_adam(nfx_ctx* c, const void* dZT, int32_t M, int32_t N, float* b, float* m, float* v, float lr_t,
                       float bc2, float beta1, float beta2, float eps, float grad_scale) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(c && dZT && b && m && v && M > 0 && N > 0, "bad argument");
     k_bias_adam<<<N, 256, 0, c->stream>>>((const __bf16*)dZT, M, b, m, v, lr_t, bc2, beta1, beta2, eps, grad_scale);
     NFX_CHECK_LAUNCH();

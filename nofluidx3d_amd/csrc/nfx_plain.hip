@@ -2016,7 +2016,7 @@ int nfx_init(int device_id, void* stream, nfx_ctx** out) {
 
 int nfx_destroy(nfx_ctx* c) {
     if (!c) return NFX_OK;
-    (void)hipSetDevice(c->device);
+    const nfx::DeviceScope device_scope(c);
     (void)hipStreamSynchronize(c->stream);
     nfx::drop_graphs(c);
     (void)hipFree(c->partials);
@@ -2039,6 +2039,7 @@ int nfx_graph_captures(nfx_ctx* c, int64_t* count) {
 }
 
 int nfx_stream_sync(nfx_ctx* c) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(c, "ctx is NULL");
     NFX_HIP(hipStreamSynchronize(c->stream));
     return NFX_OK;
@@ -2055,6 +2056,7 @@ int nfx_device_name(nfx_ctx* c, char* buf, int32_t len) {
 int nfx_batch_geometry(nfx_ctx* c, const double* p_rel, const double* cell_scale, const uint32_t* node_cell,
                        const uint32_t* tetras, const uint16_t* tile_ntet, int32_t tile_k, int64_t N, int64_t T,
                        float* ref, float* dminv, float* v0) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(c && p_rel && cell_scale && node_cell && tetras && tile_ntet && ref && dminv && v0, "NULL argument");
     NFX_REQUIRE(tile_k == 128 || tile_k == 256 || tile_k == 512, "tile_k must be 128, 256 or 512");
     int rc = check_sizes(N, T);
@@ -2070,6 +2072,7 @@ int nfx_batch_geometry(nfx_ctx* c, const double* p_rel, const double* cell_scale
 
 int nfx_precompute_f64(nfx_ctx* c, const double* edge_vectors, const double* volumes, int64_t T, float* dminv,
                        float* v0) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(c && edge_vectors && volumes && dminv && v0, "NULL argument");
     NFX_REQUIRE(T > 0 && T < (int64_t(1) << 30), "tetra count %lld out of range", (long long)T);
     k_precompute_f64<<<nblocks(T), kBlock, 0, c->stream>>>(edge_vectors, volumes, T, dminv, v0);
@@ -2106,6 +2109,7 @@ static int tetra_common(nfx_ctx* c, const nfx_elastic* m, const float* points, c
 int nfx_legacy_force(nfx_ctx* c, const nfx_elastic* m, const float* points, const uint32_t* tetras,
                      const float* dminv, int64_t N, int64_t T, float* von_mises, float* pressure, float* force,
                      float* corners) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(c && m && points && tetras && dminv && (force || corners), "NULL argument");
     NFX_REQUIRE(is_legacy(m->model), "not a legacy law: model %d", m->model);
     int rc = check_sizes(N, T);
@@ -2121,12 +2125,14 @@ int nfx_legacy_force(nfx_ctx* c, const nfx_elastic* m, const float* points, cons
 
 int nfx_tetra_force(nfx_ctx* c, const nfx_elastic* m, const float* points, const uint32_t* tetras, const float* dminv,
                     const float* v0, int64_t N, int64_t T, float* force) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(force, "force is NULL");
     return tetra_common(c, m, points, tetras, dminv, v0, N, T, force, nullptr);
 }
 
 int nfx_tetra_corner_forces(nfx_ctx* c, const nfx_elastic* m, const float* points, const uint32_t* tetras,
                             const float* dminv, const float* v0, int64_t N, int64_t T, float* corners) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(corners, "corners is NULL");
     return tetra_common(c, m, points, tetras, dminv, v0, N, T, nullptr, corners);
 }
@@ -2134,6 +2140,7 @@ int nfx_tetra_corner_forces(nfx_ctx* c, const nfx_elastic* m, const float* point
 int nfx_viscoplastic_force(nfx_ctx* c, const nfx_viscoplastic* vp, const float* points, const uint32_t* tetras,
                            const float* dminv, int64_t N, int64_t T, float* Fp, float* epsbar, float* von_mises,
                            float* pressure, float* force, float* corners) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(c && vp && points && tetras && dminv && Fp && epsbar && (force || corners), "NULL argument");
     int rc = check_sizes(N, T);
     if (rc) return rc;
@@ -2146,6 +2153,7 @@ int nfx_viscoplastic_force(nfx_ctx* c, const nfx_viscoplastic* vp, const float* 
 }
 
 int nfx_vp_q_from_fp(nfx_ctx* c, const float* Fp, int64_t T, float* Q) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(c && Fp && Q, "NULL argument");
     NFX_REQUIRE(T > 0 && T < (int64_t(1) << 30), "tetra count %lld out of range", (long long)T);
     k_vp_convert<true><<<nblocks(T), kBlock, 0, c->stream>>>(Fp, T, Q);
@@ -2154,6 +2162,7 @@ int nfx_vp_q_from_fp(nfx_ctx* c, const float* Fp, int64_t T, float* Q) {
 }
 
 int nfx_vp_fp_from_q(nfx_ctx* c, const float* Q, int64_t T, float* Fp) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(c && Q && Fp, "NULL argument");
     NFX_REQUIRE(T > 0 && T < (int64_t(1) << 30), "tetra count %lld out of range", (long long)T);
     k_vp_convert<false><<<nblocks(T), kBlock, 0, c->stream>>>(Q, T, Fp);
@@ -2162,6 +2171,7 @@ int nfx_vp_fp_from_q(nfx_ctx* c, const float* Q, int64_t T, float* Fp) {
 }
 
 int nfx_vp_tile_flags(nfx_ctx* c, const nfx_plan* p) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(c && p, "NULL argument");
     const int rc = validate_plan(p);
     if (rc) return rc;
@@ -2175,6 +2185,7 @@ int nfx_vp_tile_flags(nfx_ctx* c, const nfx_plan* p) {
 }
 
 int nfx_points_from_disp(nfx_ctx* c, const float* ref, const float* disp, int64_t N, float* points) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(c && ref && disp && points, "NULL argument");
     NFX_REQUIRE(N > 0 && N < (int64_t(1) << 31), "node count out of range");
     k_disp_convert<true><<<nblocks(3 * N), kBlock, 0, c->stream>>>(ref, disp, 3 * N, points);
@@ -2183,6 +2194,7 @@ int nfx_points_from_disp(nfx_ctx* c, const float* ref, const float* disp, int64_
 }
 
 int nfx_disp_from_points(nfx_ctx* c, const float* ref, const float* points, int64_t N, float* disp) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(c && ref && disp && points, "NULL argument");
     NFX_REQUIRE(N > 0 && N < (int64_t(1) << 31), "node count out of range");
     k_disp_convert<false><<<nblocks(3 * N), kBlock, 0, c->stream>>>(ref, points, 3 * N, disp);
@@ -2192,6 +2204,7 @@ int nfx_disp_from_points(nfx_ctx* c, const float* ref, const float* points, int6
 
 int nfx_gather_corners(nfx_ctx* c, const uint32_t* off, const uint32_t* slots, const float* corners, int64_t N,
                        float* force) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(c && off && slots && corners && force, "NULL argument");
     NFX_REQUIRE(N > 0 && N < (int64_t(1) << 31), "node count out of range");
     NodeArgs a{};
@@ -2340,6 +2353,7 @@ int nfx_order_tiles_host(int64_t ntiles, int32_t K, int32_t MX, const uint32_t* 
 }
 
 int nfx_sphere_force(nfx_ctx* c, float* force, const float* points, int64_t N, double k, double radius, double pos) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(c && force && points && N > 0, "bad argument");
     k_sphere<<<nblocks(N), kBlock, 0, c->stream>>>(force, points, N, (float)k, (float)radius, (float)pos);
     NFX_CHECK_LAUNCH();
@@ -2347,6 +2361,7 @@ int nfx_sphere_force(nfx_ctx* c, float* force, const float* points, int64_t N, d
 }
 
 int nfx_substrate_force(nfx_ctx* c, float* force, const float* points, int64_t N, double k, double wall) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(c && force && points && N > 0, "bad argument");
     k_substrate<<<nblocks(N), kBlock, 0, c->stream>>>(force, points, N, (float)k, (float)wall);
     NFX_CHECK_LAUNCH();
@@ -2354,6 +2369,7 @@ int nfx_substrate_force(nfx_ctx* c, float* force, const float* points, int64_t N
 }
 
 int nfx_plane_force(nfx_ctx* c, float* force, const float* points, int64_t N, double k, double wall) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(c && force && points && N > 0, "bad argument");
     k_plane<<<nblocks(N), kBlock, 0, c->stream>>>(force, points, N, (float)k, (float)wall);
     NFX_CHECK_LAUNCH();
@@ -2361,6 +2377,7 @@ int nfx_plane_force(nfx_ctx* c, float* force, const float* points, int64_t N, do
 }
 
 int nfx_velocity_verlet(nfx_ctx* c, float* points, float* vel, float* force, float* fold, int64_t N, int32_t fix) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(c && points && vel && force && fold && N > 0, "bad argument");
     k_vv<<<nblocks(N), kBlock, 0, c->stream>>>(points, vel, force, fold, N, fix);
     NFX_CHECK_LAUNCH();
@@ -2369,6 +2386,7 @@ int nfx_velocity_verlet(nfx_ctx* c, float* points, float* vel, float* force, flo
 
 int nfx_tip_force(nfx_ctx* c, const float* points, const float* ref, int64_t N, int32_t ind, double k, double radius,
                   double pos, double* out2) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(c && points && out2 && N > 0, "bad argument");
     NFX_REQUIRE(ind == NFX_INDENTER_SPHERE || ind == NFX_INDENTER_PLANE, "unknown indenter %d", ind);
     const unsigned int nb = std::min<unsigned int>(nblocks(N), kMaxReduceBlocks);
@@ -2430,6 +2448,7 @@ int nfx_tip_force_noalloc(const float* points, const float* ref, int64_t N, int3
 }
 
 int nfx_node_update(nfx_ctx* c, const nfx_plan* p, int64_t step, double* tip_out) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(c, "ctx is NULL");
     int rc = validate_plan(p);
     if (rc) return rc;
@@ -2438,6 +2457,7 @@ int nfx_node_update(nfx_ctx* c, const nfx_plan* p, int64_t step, double* tip_out
 }
 
 int nfx_run_steps(nfx_ctx* c, const nfx_plan* p, int64_t step0, int64_t nsteps, double* tip_hist, int32_t use_graph) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(c, "ctx is NULL");
     int rc = validate_plan(p);
     if (rc) return rc;
@@ -2493,6 +2513,7 @@ int nfx_run_steps(nfx_ctx* c, const nfx_plan* p, int64_t step0, int64_t nsteps, 
 }
 
 int nfx_time_passes(nfx_ctx* c, const nfx_plan* p, int64_t step0, int32_t nrep, double* ms_force, double* ms_node) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(c && ms_force && ms_node && nrep > 0, "bad argument");
     int rc = validate_plan(p);
     if (rc) return rc;
@@ -2564,6 +2585,7 @@ int nfx_time_passes(nfx_ctx* c, const nfx_plan* p, int64_t step0, int32_t nrep, 
 
 int nfx_batch_run_steps(nfx_ctx* c, const nfx_plan* p, const nfx_batch* b, int64_t step0, int64_t nsteps,
                         int32_t use_graph) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(c, "ctx is NULL");
     int rc = validate_plan(p);
     if (rc) return rc;
@@ -2595,6 +2617,7 @@ int nfx_batch_run_steps(nfx_ctx* c, const nfx_plan* p, const nfx_batch* b, int64
 
 int nfx_batch_time_passes(nfx_ctx* c, const nfx_plan* p, const nfx_batch* b, int64_t step0, int32_t nrep,
                           double* ms_force, double* ms_node, double* ms_curve) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(c && ms_force && ms_node && ms_curve && nrep > 0, "bad argument");
     int rc = validate_plan(p);
     if (rc) return rc;
@@ -2633,6 +2656,7 @@ int nfx_batch_time_passes(nfx_ctx* c, const nfx_plan* p, const nfx_batch* b, int
 
 
 int nfx_stream_copy(nfx_ctx* c, const void* src, void* dst, int64_t bytes, int32_t nrep, double* ms) {
+    NFX_ON_DEVICE(c);
     NFX_REQUIRE(c && src && dst && ms && nrep > 0 && bytes > 0 && bytes % 16 == 0, "bad argument");
     const int64_t n4 = bytes / 16;
     NFX_REQUIRE((n4 + kBlock - 1) / kBlock < (int64_t(1) << 31), "copy too large");
