@@ -107,21 +107,12 @@ def sync(sim):
     torch.cuda.synchronize()
 
 
-def graph_captures():
-    import ctypes
-
-    from nofluidx3d_amd import _lib, openCL
-
-    n = ctypes.c_int64()
-    _lib.call("nfx_graph_captures", openCL.handle(), ctypes.byref(n))
-    return n.value
-
-
 def time_steps(sim, warmup, steps):
-    """ms per step over ``steps`` steps, after a first call of the same length (which captures the
-    graph blocks the timed call replays) and ``warmup`` more steps; returns (s/step, captures in the
-    timed region)"""
-    sim.advance(steps)
+    """ms per step over ``steps`` steps, after calls of the same length (which capture the graph blocks
+    the timed call replays) and ``warmup`` more steps; returns (s/step, captures in the timed region)"""
+    from nofluidx3d_amd.autotune import graph_captures, warm_up
+
+    warm_up(sim, steps)
     sim.advance(warmup)
     sync(sim)
     c0 = graph_captures()
@@ -196,7 +187,7 @@ def bench_batched(steps=10000, ncells=512, form="auto", log=log):
     cell; tile size, cache policy and cell grouping from the autotuner (``form`` "auto"), or fixed:
     "groups" (cache-sized cell groups, tile 256, default policy) or "single" (one batch, tile 256,
     nontemporal).  Returns the JSON block."""
-    from nofluidx3d_amd.autotune import group_tetra, tune_batch
+    from nofluidx3d_amd.autotune import graph_captures, group_tetra, tune_batch
     from nofluidx3d_amd.batch import CellGroups, make_meshes, sample_batch
 
     specs, stats = sample_batch(ncells, seed0=1000, steps=steps)
@@ -211,7 +202,7 @@ def bench_batched(steps=10000, ncells=512, form="auto", log=log):
         best, tuned = {"tile_k": 256, "stream_nt": 1, "group_tetra": 0}, None
     b = CellGroups(specs, meshes, max_tetra=best.get("group_tetra") or None, steps=steps, ncurve=256,
                    tile_k=best["tile_k"], stream_nt=best["stream_nt"])
-    b.advance(100)  # captures every group's 100-step graph; the groups keep them
+    b.advance(100)  # captures every group's block of steps; the groups keep them
     b.sync()
     c0 = graph_captures()
     t0 = time.perf_counter()

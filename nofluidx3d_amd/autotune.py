@@ -14,7 +14,6 @@ Tunables:
   from step to step under the default policy; a larger one streams faster past it;
 - the step form (single cells): node-fused (the node update of each step rides in the next force
   pass: one launch per step) or two launches per step;
-- ``graph_steps``: steps per captured hipGraph replay block (the library captures at most 100);
 - ``group_tetra`` (batches): run the cells as consecutive groups of at most this many tetra, each
   group all its steps before the next (``batch.CellGroups``), so that a group's working set stays
   in the memory-side cache from step to step; 0 = one batch.
@@ -22,9 +21,12 @@ Tunables:
 
 from __future__ import annotations
 
+import ctypes
 import json
 import os
 import time
+
+from nofluidx3d_amd import _lib, openCL
 
 TILE_CANDIDATES = (256, 512)
 # a single cell also tries 128-tetra tiles when 512-tetra tiles would leave the chip's 256 CUs idle
@@ -100,10 +102,26 @@ def _store(key, value):
         pass
 
 
+def graph_captures():
+    """blocks of steps that the library has captured so far"""
+    n = ctypes.c_int64()
+    _lib.call("nfx_graph_captures", openCL.handle(), ctypes.byref(n))
+    return n.value
+
+
+def warm_up(sim, nsteps):
+    """Steps a cell in calls of ``nsteps`` until the next such call captures nothing: a call of several blocks of
+    replayed steps captures the first time, a call of one block the second time"""
+    before = graph_captures()
+    sim.advance(nsteps)
+    if graph_captures() == before:
+        sim.advance(nsteps)
+
+
 def _time_steps(b, nsteps):
     """ms per step of ``nsteps`` graph-replayed steps of a batch, or of cell groups summed over the
-    groups: each group warms up (100 steps, capturing its graph) right before its own timed steps,
-    as it runs all its steps in one call in use (the library caches one batch graph at a time)"""
+    groups: each group warms up (100 steps, which capture its block) right before its own timed steps,
+    as it runs all its steps in one call in use"""
     total = 0.0
     for part in getattr(b, "groups", [b]):
         part.advance(100)
@@ -166,15 +184,13 @@ def tune_batch(specs, meshes, steps, ncurve=256, nsteps=300, use_cache=True, log
 
 def tune_simulation(sim, nsteps=300, log=None):
     """Pick ``tile_k``, ``stream_nt`` and the step form for a single-cell Simulation with the tiled
-    scatter: each candidate runs ``nsteps`` steps to capture its graph, then ``nsteps`` graph-replayed
-    steps timed on the host clock, launch costs included (what a run of the cell pays per step).
+    scatter: each candidate warms up in calls of ``nsteps`` steps (``warm_up``), then runs ``nsteps`` more,
+    timed on the host clock, launch costs included (what a run of the cell pays per step).
     The step forms are the node-fused one (one launch per step, when the plan admits it and
     ``sim.fuse_node_pass`` is not False) and two launches per step.  The state is restored afterwards.
     Sets ``sim.tile_k``, ``sim.stream_nt`` and ``sim.fuse_node_pass``; returns ((tile_k, stream_nt),
     {label: ms_per_step}) with labels "256", "256nt", ... and an "f" suffix for the node-fused form."""
     import torch
-
-    from nofluidx3d_amd import _lib, openCL
 
     if sim.scatter != "tiled":
         return (sim.tile_k, sim.stream_nt), {}
@@ -198,7 +214,7 @@ def tune_simulation(sim, nsteps=300, log=None):
                     break
                 if fused and not p.disp_b:  # the plan cannot take the node-fused form
                     continue
-                sim.advance(nsteps)
+                warm_up(sim, nsteps)
                 _lib.call("nfx_stream_sync", openCL.handle())
                 t0 = time.perf_counter()
                 sim.advance(nsteps)

@@ -78,3 +78,25 @@ def test_call_of_one_block_under_the_callers_capture(ctx):
     ref.advance(100)
     assert np.array_equal((sim.displacement * 1.0).cpu().numpy(), (ref.displacement * 1.0).cpu().numpy())
     _lib.call("nfx_destroy", h)
+
+
+@pytest.mark.parametrize("steps", [20, 120, 2 * BLOCK + 3])
+def test_timed_calls_capture_nothing(ctx, steps):
+    """the benchmark's timed call and the tuner's, of less than a block of replayed steps, one and two"""
+    import bench
+    from nofluidx3d_amd import autotune
+
+    assert bench.time_steps(build_sim(scatter="tiled"), 30, steps)[1] == 0
+    sim = build_sim(scatter="tiled")
+    advance, new = sim.advance, []
+
+    def counted(n):
+        before = captures(ctx)
+        advance(n)
+        new.append(captures(ctx) - before)
+
+    sim.advance = counted
+    times = autotune.tune_simulation(sim, nsteps=steps)[1]
+    # a candidate's calls: one or two of warm-up, the last one timed
+    assert len(new) in (2 * len(times), 3 * len(times))
+    assert not any(new[len(new) // len(times) - 1::len(new) // len(times)])
