@@ -133,6 +133,13 @@ def _time_steps(b, nsteps):
     return total
 
 
+def _batch_key(specs, tetra):
+    """cache key of a population's choice: what it is, and the step forms and groups the choice was made among (the
+    leading number counts changes of the batch's step itself)"""
+    return (f"batch5:{len(specs)}:{tetra}:{specs[0].viscosity_si is not None}:one launch to {BATCH_NODE_FUSED_MAX_TETRA}"
+            f":groups of {group_tetra()}")
+
+
 def tune_batch(specs, meshes, steps, ncurve=256, nsteps=300, use_cache=True, log=None):
     """Pick ``tile_k``, ``stream_nt`` and ``group_tetra`` for a population of cells by timing
     ``nsteps`` graph-replayed steps per candidate (the way the population then runs, launch costs
@@ -143,7 +150,7 @@ def tune_batch(specs, meshes, steps, ncurve=256, nsteps=300, use_cache=True, log
     from nofluidx3d_amd.batch import BatchSimulation, CellGroups
 
     tetra = sum(len(m[1]) for m in meshes)
-    key = f"batch4:{len(specs)}:{tetra}:{specs[0].viscosity_si is not None}"
+    key = _batch_key(specs, tetra)
     if use_cache:
         hit = _load().get(key)
         if hit:

@@ -472,3 +472,35 @@ def test_narrow_tile_arrays_round_trip():
         assert np.array_equal(h["tile_dst_base"][c] + d16[c, :k].astype(np.uint32), dst[c, :k])
     nodes[3, count[3] - 1] = nodes[3, 0] + 70000  # an offset beyond 16 bits
     assert narrow_tile_arrays(nodes.reshape(-1), dst.reshape(-1), count, MX) == {}
+
+
+def test_tuned_batch_choices_belong_to_the_step_forms_they_were_timed_in(monkeypatch, tmp_path):
+    from nofluidx3d_amd import autotune, batch
+
+    timed = []
+
+    class Timed:
+        def __init__(self, specs, meshes, tile_k=256, **kw):
+            timed.append(tile_k)
+            self.plan = type("Plan", (), {})()
+
+        def advance(self, n):
+            pass
+
+        sync = lambda self: None  # noqa: E731
+
+    monkeypatch.setattr(batch, "BatchSimulation", Timed)
+    monkeypatch.setenv("NFX_TUNE_CACHE", str(tmp_path / "tune.json"))
+    specs = [batch.CellSpec(5.0, 0.5, i, 500.0, 0.4, None, 2.0, 3.0) for i in range(3)]
+    meshes = [(np.zeros((4, 3)), np.zeros((1000, 4), int))] * 3
+    tune = lambda: autotune.tune_batch(specs, meshes, 100, nsteps=1)  # noqa: E731
+    tune()
+    assert len(timed) == len(autotune.TILE_CANDIDATES)
+    tune()
+    assert len(timed) == len(autotune.TILE_CANDIDATES)  # from the cache
+    monkeypatch.setattr(autotune, "BATCH_NODE_FUSED_MAX_TETRA", 1000)
+    tune()
+    assert len(timed) == 2 * len(autotune.TILE_CANDIDATES)
+    monkeypatch.setattr(autotune, "RESIDENT_BYTES_PER_TETRA", 57)
+    tune()
+    assert len(timed) == 3 * len(autotune.TILE_CANDIDATES)
