@@ -394,7 +394,9 @@ int nfx_node_update(nfx_ctx* ctx, const nfx_plan* plan, int64_t step, double* ti
  *      the substrate/indenter flags select the terms; their values come from the cell table). ---- */
 int nfx_batch_run_steps(nfx_ctx* ctx, const nfx_plan* plan, const nfx_batch* batch, int64_t step0, int64_t nsteps,
                         int32_t use_graph);
-/* average device time of the three batched passes over nrep steps (ms), HIP events */
+/* average device time of the three batched passes over nrep steps (ms), HIP events.  For a plan with the node-fused
+ * buffers and nrep >= 3, ms_force is the average node-fused launch over the middle steps (samples included), ms_node
+ * the call's last node pass and ms_curve the last step's samples */
 int nfx_batch_time_passes(nfx_ctx* ctx, const nfx_plan* plan, const nfx_batch* batch, int64_t step0, int32_t nrep,
                           double* ms_force, double* ms_node, double* ms_curve);
 

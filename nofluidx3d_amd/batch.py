@@ -537,6 +537,8 @@ class BatchSimulation:
         torch.cuda.synchronize()
 
     def time_passes(self, nrep=20):
+        """ms of the force, node and curve passes, over ``nrep`` steps; of a batch in the node-fused form (and at least
+        three steps) ms of its one launch per step, of a call's last node pass and of the last step's samples"""
         from nofluidx3d_amd import openCL
 
         f, n, c = ctypes.c_double(), ctypes.c_double(), ctypes.c_double()
@@ -661,7 +663,7 @@ class CellGroups:
         self._collect()
 
     def time_passes(self, nrep=20):
-        """per-step ms of the force, node and curve passes, summed over the groups"""
+        """ms of the groups' passes (``BatchSimulation.time_passes``), summed over the groups"""
         t = np.array([g.time_passes(nrep) for g in self.groups])
         return tuple(float(v) for v in t.sum(axis=0))
 

@@ -2625,6 +2625,42 @@ int nfx_batch_time_passes(nfx_ctx* c, const nfx_plan* p, const nfx_batch* b, int
     if (rc) return rc;
     std::vector<hipEvent_t> ev(4 * (size_t)nrep);
     for (auto& e : ev) NFX_HIP(hipEventCreate(&e));
+    if (node_fused(*p) && nrep >= 3) {
+        // the launches of run_fused_batch, as nfx_time_passes: launch k between ev[k] and ev[k + 1], then the last
+        // step's samples and the last node pass
+        rc = launch_batch_step(c, *p, *b, step0, nullptr, 0, 2);
+        for (int k = 1; k < nrep && rc == NFX_OK; ++k) {
+            NFX_HIP(hipEventRecord(ev[k], c->stream));
+            rc = launch_batch_fused(c, *p, *b, fused_io(*p, k, nullptr, step0 + k - 1, nullptr, 0));
+        }
+        const NodeIO io = fused_last_io(*p, nrep);
+        if (rc == NFX_OK) {
+            NFX_HIP(hipEventRecord(ev[nrep], c->stream));
+            if (b->curves) rc = launch_batch_curves(c, *p, *b, io.x, step0 + nrep - 1, nullptr, 0);
+        }
+        if (rc == NFX_OK) {
+            NFX_HIP(hipEventRecord(ev[nrep + 1], c->stream));
+            rc = launch_batch_nodes(c, *p, *b, io, step0 + nrep - 1, nullptr, 0);
+        }
+        if (rc == NFX_OK) {
+            NFX_HIP(hipEventRecord(ev[nrep + 2], c->stream));
+            NFX_HIP(hipEventSynchronize(ev[nrep + 2]));
+            double sf = 0;
+            for (int k = 2; k < nrep; ++k) {
+                float a = 0;
+                NFX_HIP(hipEventElapsedTime(&a, ev[k], ev[k + 1]));
+                sf += a;
+            }
+            float sample = 0, node = 0;
+            NFX_HIP(hipEventElapsedTime(&sample, ev[nrep], ev[nrep + 1]));
+            NFX_HIP(hipEventElapsedTime(&node, ev[nrep + 1], ev[nrep + 2]));
+            *ms_force = sf / (nrep - 2);
+            *ms_node = node;
+            *ms_curve = sample;
+        }
+        for (auto& e : ev) (void)hipEventDestroy(e);
+        return rc;
+    }
     for (int i = 0; i < nrep && rc == NFX_OK; ++i) {
         NFX_HIP(hipEventRecord(ev[4 * i], c->stream));
         rc = launch_batch_step(c, *p, *b, step0 + i, nullptr, 0, 1);

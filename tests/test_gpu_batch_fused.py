@@ -80,3 +80,28 @@ def test_curves_do_not_depend_on_the_split_into_calls(ctx, monkeypatch, tile_k):
     assert (whole[:, 200:] > 0).all()
     for limit, calls in ((0, [7] * 57 + [1]), (10 ** 9, [400]), (10 ** 9, [7] * 57 + [1]), (10 ** 9, [2] * 200)):
         assert np.array_equal(run(limit, calls), whole)
+
+
+@pytest.mark.parametrize("nrep", [1, 2, 3, 8])
+def test_timed_passes_are_those_of_the_step_form(ctx, nrep):
+    """time_passes on a batch in the node-fused form runs that form (its second buffers are written) from three steps on,
+    and advances the batch as the same number of steps does"""
+    import torch
+
+    from nofluidx3d_amd.batch import BatchSimulation, CellSpec, make_meshes
+
+    specs = [CellSpec(3.0, 0.5, 3300 + i, 500.0, 0.4, 60.0, 5.0, 3.0, indent_frac=0.5) for i in range(2)]
+    meshes = make_meshes(specs, workers=1, cache=None)
+    b, want = (BatchSimulation(specs, meshes, steps=100, ncurve=100) for _ in range(2))
+    assert b.plan.disp_b
+    b.advance(60)
+    b.sync()
+    before = b.x_b.clone()
+    times = b.time_passes(nrep)
+    want.advance(60)
+    want.advance(nrep)
+    for s, t in ((b.x, want.x), (b.v, want.v), (b.state, want.state)):
+        assert torch.equal(s, t)
+    assert np.array_equal(b.curves_sim(), want.curves_sim()) and b.curves_sim()[:, 59 + nrep].all()
+    assert all(t > 0.0 for t in times)
+    assert torch.equal(b.x_b, before) == (nrep < 3)
