@@ -278,7 +278,11 @@ __global__ __launch_bounds__(kB) void k_lve(float* __restrict__ f, float* __rest
     const float tr = e[0][0] + e[1][1] + e[2][2];
     // the state in planes of nine entries, each plane's loads together and the next term's issued before this
     // one is stored: nterms + 1 memory rounds in flight instead of 9 (nterms + 1) one after another
-    float old[9], h[9], rate[9], sig[3][3];
+    float old[9], h[9], rate[9], sig[3][3], t3;
+    {
+#pragma clang fp contract(off)
+        t3 = tr * (1.0f / 3.0f);
+    }
 #pragma unroll
     for (int q = 0; q < 9; ++q) old[q] = dev_old[q * T + t];
     if (c.nterms) {
@@ -290,8 +294,9 @@ __global__ __launch_bounds__(kB) void k_lve(float* __restrict__ f, float* __rest
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
             const int q = 3 * i + k;
-            // fused by name, so that the three axes are rounded alike whatever the compiler makes of them
-            const float dv = i == k ? __builtin_fmaf(tr, -1.0f / 3.0f, e[i][k]) : e[i][k];
+            // the trace's third is rounded on its own but in the first entry: the results of the form with one
+            // loop over the terms per entry, bit for bit
+            const float dv = i != k ? e[i][k] : i == 0 ? __builtin_fmaf(tr, -1.0f / 3.0f, e[i][k]) : e[i][k] - t3;
             rate[q] = dv - old[q];
             dev_old[q * T + t] = dv;
             sig[i][k] = c.two_mu_inf * dv + (i == k ? c.kappa * tr : 0.0f);

@@ -262,38 +262,6 @@ def test_linear_viscoelastic_steps(ctx, mesh):
     rel_close(host(tr_d), tr_r, 1e-4)
 
 
-def test_linear_viscoelastic_law_treats_the_axes_alike(ctx):
-    """one tetra stretched along x, along y and along z: the same deviator and transient stresses, bit for bit,
-    with the axes exchanged"""
-    import torch
-
-    from nofluidx3d_amd import _lib
-
-    n = 2000
-    s = np.random.default_rng(3).uniform(0.8, 1.2, n).astype(np.float32)
-    x = np.zeros((3, n, 4, 3), np.float32)  # axis, tetra, corner, component: edges e_x, e_y, e_z from a corner at 0
-    x[:, :, 1:] = np.eye(3, dtype=np.float32)
-    for i in range(3):
-        x[i, :, 1 + i, i] = s
-    nT = 3 * n
-    P = _lib.Viscoelastic()
-    P.E, P.nu, P.nterms, P.weights[0], P.taus[0] = 0.01, 0.42, 1, 0.3, 5.0
-    xd = dev(x.reshape(-1, 3).reshape(-1, order="F"), np.float32)
-    td = dev(O.soa(np.arange(4 * nT).reshape(-1, 4), np.uint32))
-    dminv = dev(np.repeat(np.eye(3).reshape(9, 1), nT, 1).reshape(-1), np.float32)
-    out = [torch.zeros(k * nT, dtype=torch.float32, device="cuda:0") for k in (9, 9, 12)]
-    call("nfx_linear_viscoelastic_force", ctx, P, xd.data_ptr(), td.data_ptr(), dminv.data_ptr(), 4 * nT, nT,
-         out[0].data_ptr(), out[1].data_ptr(), None, None, None, out[2].data_ptr())
-    for o in out[:2]:
-        d = host(o).reshape(3, 3, 3, n)  # row, column, axis of the stretch, tetra
-        assert (d[0, 0, 0] != 0).all()
-        for i in (1, 2):
-            assert np.array_equal(d[i, i, i], d[0, 0, 0])
-            for k in range(3):
-                if k != i:
-                    assert np.array_equal(d[k, k, i], d[1, 1, 0])
-
-
 def test_hard_adhesive_setter_through_simulation(ctx):
     """setInteractionHardAdhesivePlaneNonDimensional (SimulationLegacy.py:657-692) on a Simulation: the
     wall 0.2 below the cell, A = AdhesionConstant E R / (p0 L0), k = PotentialForceConst; one enqueue
