@@ -202,8 +202,9 @@ typedef struct {
     int32_t ncurve;
     int64_t curve_steps; /* sample k is taken at the first step s with floor(s*ncurve/curve_steps) == k */
     /* nullable, all four or none: the tile-node ids and partial positions as 16-bit offsets from
-     * per-tile bases (a tile never leaves its cell; every offset below 65536), which the force pass
-     * then reads in place of plan.tile_nodes and plan.tile_dst */
+     * per-tile bases (a tile never leaves its cell; every offset below 65536), which the force pass of a
+     * two-launch step then reads in place of plan.tile_nodes and plan.tile_dst.  Node-fused launches read the
+     * plan's 32-bit arrays, and so does a two-launch step on the nine-plane viscoplastic state */
     const uint16_t* tile_nodes16;   /* ntiles*MX: tile_nodes - tile_node_base[tile] */
     const uint16_t* tile_dst16;     /* ntiles*MX: tile_dst - tile_dst_base[tile] (padding 0) */
     const uint32_t* tile_node_base; /* ntiles */

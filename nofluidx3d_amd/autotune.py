@@ -47,14 +47,15 @@ def default_stream_nt(tetra):
 
 # the node-fused step (one launch per step) wins where launches dominate a step; on a mesh of
 # millions of tetra its force pass, which then also updates every node it touches (~2.9 times per
-# node), is longer than the two passes apart.  Measured on MI355X (NH cells, best tile shape of each
-# form, us per graph-replayed step, fused against two launches): 25k tetra 5.5 / 7.2, 106k 6.3 / 7.9,
-# 211k 7.5 / 8.8, 526k 11.7 / 12.5, 878k 16.6 / 16.5; the 3.4M-tetra viscoplastic cell 58 / 50
+# node), is longer than the two passes apart.  Measured on MI355X (lattice cells, best tile shape of each
+# form, us per graph-replayed step, fused against two launches): Neo-Hookean 20k tetra 4.7 / 6.5, 89k 5.5 / 7.0,
+# 179k 6.6 / 7.6, 0.5M 10.3 / 10.1, 0.84M 13.8 / 13.8, 2.6M 31.0 / 30.5; with yield 0.5M 11.9 / 11.9, 0.84M 15.8 / 15.0,
+# 2.6M 36.4 / 34.5; with hardening flow 0.5M 15.6 / 16.1, 0.84M 23.7 / 23.5, 2.6M 57.7 / 54.0
 NODE_FUSED_MAX_TETRA = 600_000
 # batches hold out longer: their node pass looks each node's cell up, and the curve samples ride in the one launch.
-# Elastic 46k 6.2 / 8.2, 234k 8.1 / 10.0, 1.4M 23.5 / 24.6, 2.5M 32.0 / 33.5, 3.8M 45.7 / 45.0; viscoplastic 46k 6.3 / 8.9,
-# 234k 9.2 / 11.5, 1.4M 30.1 / 35.1, 2.3M 46.5 / 48.1, 2.5M 49.3 / 51.8, 3.8M 85.3 / 75.1 (cells of 10 k to 100 k tetra,
-# 256-tetra tiles, 43 % of the steps with samples from 1.4M on)
+# Viscoplastic 46k 5.7 / 8.9, 0.19M 7.8 / 10.5, 1.4M 28.0 / 35.6, 2.7M 48.7 / 52.7, 3.5M 77.5 / 61.3 (cells of 4 k to 150 k
+# tetra, 256-tetra tiles, 43 % of the steps with samples); elastic batches gain at every size measured: 46k 5.7 / 8.4,
+# 0.19M 7.1 / 9.2, 1.4M 22.5 / 28.5, 2.7M 32.8 / 43.0, 3.5M 39.6 / 47.4, 4.8M 53.7 / 57.3 (the line is the viscoplastic ones')
 BATCH_NODE_FUSED_MAX_TETRA = 2_600_000
 
 

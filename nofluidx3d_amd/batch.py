@@ -342,7 +342,7 @@ class BatchSimulation:
     ``stream_nt`` cache policy of the force pass's streams (None: nontemporal beyond the 256 MB
     memory-side cache); ``sym_state`` viscoplastic state Gd = Fp^-1 Fp^-T - I (6 floats) instead of
     Q = Fp^-1 - I (9);
-    ``narrow`` 16-bit tile-node ids and partial positions (when every cell has < 65536 nodes);
+    ``narrow`` 16-bit tile-node ids and partial positions (when every cell has < 65536 nodes), read by two-launch steps;
     ``shape_from_ref`` the force pass forms Dm^-1 from the reference positions instead of streaming it.
     Batches of at most ``autotune.BATCH_NODE_FUSED_MAX_TETRA`` tetra run the node-fused step (same bits).
 

@@ -44,9 +44,10 @@ void set_error(const char* fmt, ...);
 
 // reduction scratch: per-block FP64 partials and a completion counter, allocated once per context
 constexpr int kMaxReduceBlocks = 2048;
-// steps per captured graph (even).  A call records every 100 steps as a rule, and its first and last steps and the one that
-// starts w are not replayed: 96 lets such a call replay one block.  A replayed step of a small cell is 0.5 us shorter than
-// one launched by the host (25 k tetra: 100 steps 521 -> 476 us), a replay costs about 5 us
+// steps per captured graph (even).  Chosen for calls of 100 steps, the recording interval of the small benchmark cell: a
+// call's first and last steps and the one that starts w are not replayed, and 96 lets such a call replay one block (a
+// shorter call replays nothing).  A replayed step of a small cell is 0.5 us shorter than one launched by the host (25 k
+// tetra: 100 steps 521 -> 476 us), a replay costs about 5 us
 constexpr int kGraphBlock = 96;
 constexpr int kMaxGraphs = 32;    // captured graphs a context keeps
 

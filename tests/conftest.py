@@ -19,3 +19,26 @@ def oracle_lib():
 
     oracle.lib()
     return oracle
+
+
+@pytest.fixture(scope="module", autouse=True)
+def own_step_blocks(request):
+    """For the modules whose tests count captured step blocks: a library context of their own, and no garbage collection
+    between their tests.  The library finds a captured block by its plan, addresses included; a simulation collected
+    in between would give its addresses to the next one, which then replays the old block instead of capturing."""
+    if request.module.__name__ not in ("test_gpu_plain", "test_gpu_graph_calls"):
+        yield
+        return
+    import gc
+
+    from nofluidx3d_amd import openCL
+
+    if openCL.context is not None:
+        openCL.getCommandQueue().finish()
+        openCL.context.release()
+        openCL.context = None
+    gc.collect()
+    gc.disable()
+    yield
+    gc.enable()
+    gc.collect()
